@@ -589,5 +589,53 @@ __device__ __forceinline__ double from_acc<double>(double v) {
   return v;
 }
 
+// Activations of the generic and register-staged paths, in AT (float, or
+// double for fp64), on values already rounded to T.
+template <typename AT>
+__device__ __forceinline__ void gelu_both(AT x, AT& y, AT& dy) {
+  const AT cdf = AT(0.5) * (AT(1) + erf(x * AT(0.70710678118654752440)));
+  const AT pdf = exp(AT(-0.5) * x * x) * AT(0.39894228040143267794);
+  y = x * cdf;
+  dy = cdf + x * pdf;
+}
+template <typename T, typename AT>
+__device__ __forceinline__ AT swiglu_fwd(AT g, AT v) {
+  const AT sg = AT(1) / (AT(1) + exp(-g));
+  const AT silu = to_acc<T>(from_acc<T>(g * sg));
+  return silu * v;
+}
+template <typename T, typename AT>
+__device__ __forceinline__ void swiglu_bwd(AT dh, AT g, AT v, AT& dg, AT& dv) {
+  const AT sg = AT(1) / (AT(1) + exp(-g));
+  const AT silu = to_acc<T>(from_acc<T>(g * sg));
+  const AT ds = to_acc<T>(from_acc<T>(dh * v));
+  dg = (ds * sg) * (AT(1) + g * (AT(1) - sg));
+  dv = dh * silu;
+}
+
+// Tile bookkeeping shared by the launchers: n-tiles, m-tile slots and the
+// grid size (one workgroup per tile).
+template <int MODE>
+int64_t plan_tiles(GemmArgs& g, int64_t out_cols, int BM, int BN) {
+  g.ntn = (int32_t)ceil_div(out_cols, BN);
+  if (MODE == kDw) {
+    g.ntm = (int32_t)ceil_div(g.K, BM);
+    // Chunks: at most one per expert plus A / chunk (upper bound).
+    const int64_t chunks = g.chunk > 0 ? g.E + g.A / g.chunk : g.E;
+    g.mtiles = chunks * g.ntm;
+  } else {
+    g.ntm = 0;
+    g.mtiles = ceil_div(g.A, BM) + g.E;  // upper bound: each expert's last tile may be partial
+  }
+  return g.mtiles * g.ntn;
+}
+
 }  // namespace
+
+// staged_gemm.hip: whether the register-staged kernel takes this GEMM, and
+// its launch (epilogue fused).
+bool staged_ok(int mode, int dtype, const GemmArgs& g);
+int launch_staged_gemm(int mode, int epi, int dtype, const GemmArgs& g, int64_t out_cols,
+                       hipStream_t s);
+
 }  // namespace nt
