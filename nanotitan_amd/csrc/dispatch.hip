@@ -226,27 +226,38 @@ pack_rows_kernel(const V* __restrict__ X, const float* __restrict__ w,
   if (base_mode == 0) {
     for (int e = tid; e < E; e += kDispatchThreads) s_base[e] = base[e];
   } else if (base_mode == 2) {
-    for (int e = wave; e < E; e += kDispatchWaves) {
-      const int32_t* h = hist + (int64_t)e * nb;
+    // A group of `seg` lanes sums one expert's row, at most eight loads per
+    // lane where 64 lanes reach that: with few blocks a wave serves many
+    // experts at once, and a launch of a few tokens waits for one round of
+    // loads and shuffles instead of one per expert (33 tokens, 128 experts:
+    // 8.6 us, 30 us with a whole wave per expert).
+    int seg = 1;
+    while (seg < kWave && 8 * seg < nb) seg <<= 1;
+    const int sl = lane & (seg - 1), per_wave = kWave / seg;
+    for (int e0 = wave * per_wave; e0 < E; e0 += kDispatchWaves * per_wave) {
+      const int e = e0 + lane / seg;
+      const int32_t* h = hist + (int64_t)min(e, E - 1) * nb;
       int tot = 0, before = 0;
       // Eight loads in flight per lane (the entries are L2-resident).
-      for (int i0 = 0; i0 < nb; i0 += 8 * kWave) {
+      for (int i0 = 0; i0 < nb; i0 += 8 * seg) {
         int v[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-          const int i = i0 + u * kWave + lane;
+          const int i = i0 + u * seg + sl;
           v[u] = i < nb ? h[i] : 0;
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-          const int i = i0 + u * kWave + lane;
+          const int i = i0 + u * seg + sl;
           tot += v[u];
           before += i < b ? v[u] : 0;
         }
       }
-      tot = wave_sum_int(tot);
-      before = wave_sum_int(before);
-      if (lane == 0) {
+      for (int o = seg / 2; o >= 1; o >>= 1) {
+        tot += __shfl_xor(tot, o, kWave);
+        before += __shfl_xor(before, o, kWave);
+      }
+      if (sl == 0 && e < E) {
         s_run[e] = tot;
         s_base[e] = before;
       }
