@@ -1421,18 +1421,50 @@ constexpr int64_t kSplitMinRed = 1024;
 // next tile's loads (C5 up-projection, K = 2048: 2568-2593 us split,
 // 2105-2118 us with every wave in the epilogue).
 bool gelu_split(int dtype, int64_t red) { return dtype == NT_BF16 && red >= 2048; }
+// Mean rows per expert up to which forward and dX launches run on 64-row
+// tiles. Measured on MI355X (us, 128-row tiles against 64-row ones; SwiGLU:
+// 256-row tiles; E experts d -> f, every expert with rows):
+//                        mean rows    8           32          48
+//   128, 2048 ->  768  up         83 ->  77   85 ->  80   87 ->  95
+//                      down       80 ->  73   83 ->  75
+//                      SwiGLU    176 -> 146  177 -> 154  183 -> 182
+//     8, 4096 -> 14336 up        169 -> 163  176 -> 168
+//                      down      218 -> 155  219 -> 156  221 -> 159
+//                      SwiGLU    444 -> 357  448 -> 373  457 -> 380
+//    16,  512 -> 2048  up       11.2 -> 9.0 11.8 -> 9.6 11.8 -> 9.7
+//                      down       26 ->  20   26 ->  20   26 ->  20
+//                      SwiGLU     26 ->  18   27 ->  18   27 ->  18
+// (5.0-6.1 TB/s of weights at the two larger layers). 256 columns where
+// that leaves more than 1.5 tiles per CU (a k-row of a tile is then 512
+// contiguous bytes: the 4096 -> 14336 up-projection runs 186 us on 128
+// columns), else 128 columns and two workgroups per CU (the 14336 -> 4096
+// down-projection runs 174 us on 256).
+constexpr int64_t kFewRows = 32, kFewRowsSwiGLU = 48;
 template <int MODE, int EPI>
 int launch_mfma_auto(int dtype, GemmArgs g, int64_t out_cols, hipStream_t s) {
   const int64_t chunks = g.chunk > 0 ? g.E + g.A / g.chunk : g.E;
   const int64_t tiles256 = MODE == kDw
                                ? chunks * ceil_div(g.K, 256) * ceil_div(out_cols, 256)
                                : ceil_div(g.A, 256) * ceil_div(out_cols, 256);
+  // Few rows per expert (decode): the weights' bytes bound the launch, so the
+  // tiles are 64 rows high and the LDS holds three stages of them.
+  const int64_t experts = std::min<int64_t>(g.E, g.A);  // that can have rows
+  const bool few_rows =
+      MODE != kDw && g.A <= (EPI == kEpiSwiGLU ? kFewRowsSwiGLU : kFewRows) * experts;
   // SwiGLU forward: 256 rows x (128 gate | 128 value) columns, waves 4 x 2,
   // so that each wave holds the gate and value tiles of the same outputs.
   if constexpr (EPI == kEpiSwiGLU) {
     (void)tiles256;
+    if (few_rows) return launch_mfma<MODE, EPI, 64, 256, 2, 2, 64, 3>(dtype, g, out_cols, s);
     return launch_mfma<MODE, EPI, 256, 256, 4, 2, 64, 2>(dtype, g, out_cols, s);
   } else {
+    if constexpr (MODE != kDw && (EPI == kEpiPlain || EPI == kEpiGelu)) {
+      if (few_rows) {
+        if (experts * ceil_div(out_cols, 256) * 2 > (int64_t)device_cus(s) * 3)
+          return launch_mfma<MODE, EPI, 64, 256, 2, 2, 64, 3>(dtype, g, out_cols, s);
+        return launch_mfma<MODE, EPI, 64, 128, 2, 2, 64, 3>(dtype, g, out_cols, s);
+      }
+    }
     if (tiles256 * 2 >= (int64_t)device_cus(s) * 3) {
       if constexpr (MODE != kDw && (EPI == kEpiPlain || EPI == kEpiDualK)) {
         const int64_t red = MODE == kFwd ? g.K : (EPI == kEpiDualK ? 2 * g.N : g.N);
