@@ -260,6 +260,33 @@ int nt_route_topk_count(const float* logits, int64_t T, int32_t E, int32_t k, fl
 int nt_route_topk_backward(const float* gates, const int32_t* topk, const float* dgates,
                            int64_t T, int32_t E, int32_t k, float* dlogits, hipStream_t stream);
 
+/* Load-balancing statistics of T >= 1 tokens (reference src/model/utils.py:77-93):
+ * total = sum of counts, frac = counts / total, mean[e] = mean over tokens of
+ * softmax(logits)[t,e], aux = coef * sum_e frac[e] * mean[e]. logits [T,E]
+ * f32, counts [E] i32. The workspace (0 bytes for few tokens) holds partial
+ * column sums. */
+size_t nt_router_stats_workspace_bytes(int64_t T, int32_t E);
+int nt_router_stats(const float* logits, const int32_t* counts, int64_t T, int32_t E, float coef,
+                    int64_t* total, float* frac, float* mean, float* aux, void* ws,
+                    size_t ws_bytes, hipStream_t stream);
+
+/* Gradient of aux and mean to the logits: dlogits [T,E]. daux (one float)
+ * and dmean [E] are device pointers; NULL means zero. */
+int nt_router_stats_backward(const float* logits, const float* frac, const float* daux,
+                             const float* dmean, int64_t T, int32_t E, float coef, float* dlogits,
+                             hipStream_t stream);
+
+/* Backward of logits = x @ W^T used twice (the gate path with gradient dl,
+ * the statistics path on detached tokens with gradient da; [T,E] f32, NULL
+ * means zero): dx = dl @ W in x's dtype, dW = (dl + da)^T @ x in f32, each
+ * skipped when NULL. x, dx [T,d] (f32, f16 or bf16), W, dW [E,d] f32,
+ * E <= 32. The workspace holds dW's partial sums. Replaces torch's backward
+ * of the two router passes of reference src/model/cuda_backend.py:27-41. */
+size_t nt_router_linear_backward_workspace_bytes(int64_t T, int32_t E, int64_t d);
+int nt_router_linear_backward(int dtype, const void* x, const float* W, const float* dl,
+                              const float* da, int64_t T, int32_t E, int64_t d, void* dx,
+                              float* dW, void* ws, size_t ws_bytes, hipStream_t stream);
+
 /* ------------------------------------------------------------- grouped GEMM */
 
 /* Workspace for nt_grouped_gemm_dw and the paired dW + dX calls with these

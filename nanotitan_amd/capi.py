@@ -9,7 +9,7 @@ signature; ``load()`` checks that the library exports all of them.
 from __future__ import annotations
 
 import ctypes
-from ctypes import c_char_p, c_int, c_int32, c_int64, c_size_t, c_uint32, c_void_p
+from ctypes import c_char_p, c_float, c_int, c_int32, c_int64, c_size_t, c_uint32, c_void_p
 from functools import lru_cache
 
 from nanotitan_amd.extension import LIB_PATH
@@ -95,6 +95,20 @@ EXPORTS: dict[str, tuple[object, list[object]]] = {
         [_P, c_int64, c_int32, c_int32, _P, _P, _P, c_int32, _P, _P],
     ),
     "nt_route_topk_backward": (c_int, [_P, _P, _P, c_int64, c_int32, c_int32, _P, _P]),
+    "nt_router_stats_workspace_bytes": (c_size_t, [c_int64, c_int32]),
+    "nt_router_stats": (
+        c_int,
+        [_P, _P, c_int64, c_int32, c_float, _P, _P, _P, _P, _P, c_size_t, _P],
+    ),
+    "nt_router_stats_backward": (
+        c_int,
+        [_P, _P, _P, _P, c_int64, c_int32, c_float, _P, _P],
+    ),
+    "nt_router_linear_backward_workspace_bytes": (c_size_t, [c_int64, c_int32, c_int64]),
+    "nt_router_linear_backward": (
+        c_int,
+        [c_int, _P, _P, _P, _P, c_int64, c_int32, c_int64, _P, _P, _P, c_size_t, _P],
+    ),
     "nt_grouped_gemm_workspace_bytes": (c_size_t, [c_int, c_int32, c_int64, c_int64, c_int64]),
     "nt_grouped_gemm": (
         c_int,

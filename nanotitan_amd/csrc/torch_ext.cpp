@@ -755,6 +755,92 @@ std::tuple<Tensor, Tensor> pack_backward_inv_route(Tensor dpX, Tensor dpw, Tenso
   return {dX, dlogits};
 }
 
+// router_stats(logits, counts, coef) -> (total i64, frac [E], mean [E], aux):
+// the load-balancing statistics of MoELayerStats.
+std::tuple<Tensor, Tensor, Tensor, Tensor> router_stats(Tensor logits, Tensor counts, double coef) {
+  check_f32(logits, "logits");
+  check_i32(counts, "counts");
+  TORCH_CHECK(logits.is_contiguous() && counts.is_contiguous(), "inputs must be contiguous");
+  TORCH_CHECK(logits.dim() == 2 && counts.numel() == logits.size(1),
+              "expected logits [T,E] and counts [E]");
+  check_same_device(logits, {&counts});
+  const int64_t T = logits.size(0), E = logits.size(1);
+  c10::hip::HIPGuard guard(logits.get_device());
+  Tensor total = at::empty({}, logits.options().dtype(at::kLong));
+  Tensor frac = at::empty({E}, logits.options());
+  Tensor mean = at::empty({E}, logits.options());
+  Tensor aux = at::empty({}, logits.options());
+  Tensor ws = workspace(logits, nt_router_stats_workspace_bytes(T, (int32_t)E));
+  check_status(nt_router_stats(logits.data_ptr<float>(), counts.data_ptr<int32_t>(), T, (int32_t)E,
+                               (float)coef, total.data_ptr<int64_t>(), frac.data_ptr<float>(),
+                               mean.data_ptr<float>(), aux.data_ptr<float>(), ws.data_ptr(),
+                               ws.numel(), stream_of(logits)),
+               "router_stats");
+  return {total, frac, mean, aux};
+}
+
+// Gradient of router_stats' aux and mean to the logits.
+Tensor router_stats_backward(Tensor logits, Tensor frac, c10::optional<Tensor> daux,
+                             c10::optional<Tensor> dmean, double coef) {
+  check_f32(logits, "logits");
+  check_f32(frac, "frac");
+  const int64_t T = logits.size(0), E = logits.size(1);
+  TORCH_CHECK(logits.is_contiguous() && frac.is_contiguous() && frac.numel() == E,
+              "expected contiguous logits [T,E] and frac [E]");
+  check_same_device(logits, {&frac});
+  for (auto& t : {std::make_pair(&daux, int64_t(1)), std::make_pair(&dmean, E)}) {
+    if (!t.first->has_value()) continue;
+    check_f32(**t.first, "grad");
+    TORCH_CHECK((*t.first)->is_contiguous() && (*t.first)->numel() == t.second,
+                "expected a contiguous gradient of aux (one value) or mean [E]");
+    check_same_device(logits, {&**t.first});
+  }
+  c10::hip::HIPGuard guard(logits.get_device());
+  Tensor out = at::empty_like(logits);
+  check_status(nt_router_stats_backward(logits.data_ptr<float>(), frac.data_ptr<float>(),
+                                        daux ? daux->data_ptr<float>() : nullptr,
+                                        dmean ? dmean->data_ptr<float>() : nullptr, T, (int32_t)E,
+                                        (float)coef, out.data_ptr<float>(), stream_of(logits)),
+               "router_stats_backward");
+  return out;
+}
+
+// router_linear_backward(x, W, dl, da, need_dx, need_dW) -> (dx, dW): dx = dl W,
+// dW = (dl + da)^T x; a missing gradient is zero, an output not needed undefined.
+std::tuple<c10::optional<Tensor>, c10::optional<Tensor>> router_linear_backward(
+    Tensor x, Tensor W, c10::optional<Tensor> dl, c10::optional<Tensor> da, bool need_dx,
+    bool need_dW) {
+  check_device(x, "x");
+  check_f32(W, "weight");
+  TORCH_CHECK(x.is_contiguous() && W.is_contiguous(), "inputs must be contiguous");
+  TORCH_CHECK(x.dim() == 2 && W.dim() == 2 && x.size(1) == W.size(1),
+              "expected x [T,d] and weight [E,d]");
+  const int64_t T = x.size(0), d = x.size(1), E = W.size(0);
+  check_same_device(x, {&W});
+  for (auto* t : {&dl, &da}) {
+    if (!t->has_value()) continue;
+    check_f32(**t, "grad");
+    TORCH_CHECK((*t)->is_contiguous() && (*t)->dim() == 2 && (*t)->size(0) == T &&
+                    (*t)->size(1) == E,
+                "expected contiguous logit gradients [T,E]");
+    check_same_device(x, {&**t});
+  }
+  c10::hip::HIPGuard guard(x.get_device());
+  c10::optional<Tensor> dx, dW;
+  if (need_dx) dx = at::empty_like(x);
+  if (need_dW) dW = at::empty_like(W);
+  Tensor ws = workspace(
+      x, need_dW ? nt_router_linear_backward_workspace_bytes(T, (int32_t)E, d) : 0);
+  check_status(nt_router_linear_backward(
+                   dtype_code(x), x.data_ptr(), W.data_ptr<float>(),
+                   dl ? dl->data_ptr<float>() : nullptr, da ? da->data_ptr<float>() : nullptr, T,
+                   (int32_t)E, d, need_dx ? dx->data_ptr() : nullptr,
+                   need_dW ? dW->data_ptr<float>() : nullptr, ws.data_ptr(), ws.numel(),
+                   stream_of(x)),
+               "router_linear_backward");
+  return {dx, dW};
+}
+
 // stream_copy(dst, src, blocks=0): the library's 16-byte streaming copy of
 // src's bytes into dst (the achievable-bandwidth reference of the benchmark).
 void stream_copy(Tensor dst, Tensor src, int64_t blocks) {
@@ -1086,6 +1172,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("dispatch_tokens_counted", &dispatch_tokens_counted,
         "dispatch_tokens from the counts route_topk_count computed");
   m.def("route_topk_backward", &route_topk_backward, "Gradient of route_topk's gates -> dlogits");
+  m.def("router_stats", &router_stats,
+        "Load-balancing statistics -> (total, frac [E], mean [E], aux)");
+  m.def("router_stats_backward", &router_stats_backward,
+        "Gradient of router_stats' aux and mean to the logits");
+  m.def("router_linear_backward", &router_linear_backward,
+        "Backward of the router's linear layer for both of its gradients -> (dx, dW)");
   m.def("stream_fill", &stream_fill, "16-byte streaming device fill (write bandwidth reference)",
         pybind11::arg("dst"), pybind11::arg("value") = 0);
   m.def("stream_read", &stream_read, "16-byte streaming device read (read bandwidth reference)",

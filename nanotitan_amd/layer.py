@@ -33,6 +33,8 @@ from nanotitan_amd.moe_ops import (
     grouped_gelu_ffn_fn,
     route_dispatch_fn,
     route_fn,
+    router_linear_fn,
+    router_stats_fn,
     swiglu_ffn_fn,
 )
 
@@ -74,6 +76,18 @@ class MoELayerStats:
             * self.cfg.num_experts
             * torch.sum(self.ass_frac_per_expert * self.probs_per_expert)
         )
+
+    @classmethod
+    def from_logits(cls, tokens_per_expert, logits, cfg):
+        """The same statistics from the float32 router logits, in one kernel."""
+        stats = cls.__new__(cls)
+        stats.tokens_per_expert = tokens_per_expert
+        stats.cfg = cfg
+        stats.num_tokens = logits.shape[0]
+        (stats.total_assignments, stats.ass_frac_per_expert, stats.probs_per_expert,
+         stats.aux_loss) = router_stats_fn(logits, tokens_per_expert,
+                                           cfg.router_alpha * cfg.num_experts)
+        return stats
 
 
 def route(logits: torch.Tensor, top_k: int):
@@ -153,6 +167,20 @@ def moe_forward_from_logits(x_flat, logits, experts, num_experts, top_k):
     return out, counts, gates
 
 
+def _plain_router(router, flat) -> bool:
+    """Whether calling ``router`` is exactly float32 ``flat @ weight.T``, with no
+    hook, subclass, cast or bias that a second call could make differ."""
+    hooks = (router._forward_hooks, router._forward_pre_hooks, router._backward_hooks,
+             router._backward_pre_hooks)
+    return (type(router) is nn.Linear and router.bias is None and not any(hooks)
+            and "forward" not in router.__dict__
+            and not nn.modules.module._has_any_global_hook()
+            and type(router.weight) is nn.Parameter and router.weight.dtype == torch.float32
+            and type(flat) is torch.Tensor and flat.is_cuda and router.weight.is_cuda
+            and flat.dtype in (torch.float32, torch.float16, torch.bfloat16)
+            and flat.shape[0] > 0 and not torch.is_autocast_enabled())
+
+
 class HIPMoEBackend:
     """Reference CUDAMoEBackend dataflow (src/model/cuda_backend.py:11-81) on the HIP path."""
 
@@ -167,16 +195,31 @@ class HIPMoEBackend:
         batch, seq_len, d_model = x.shape
         flat = x.reshape(-1, d_model)
         router_dtype = self.router.weight.dtype
+        plain = (_plain_router(self.router, flat)
+                 and type(self.cfg.router_alpha * self.cfg.num_experts) in (int, float))
         with record_function("moe/router"):
-            logits = self.router(flat.to(router_dtype))
-        # Aux-loss probabilities from a second router pass on detached tokens
-        # (src/model/cuda_backend.py:40-41), so the aux grad reaches only the router.
-        aux_probs = self.router(flat.detach().to(router_dtype)).softmax(dim=-1)
+            # Aux-loss logits from a second router pass on detached tokens
+            # (src/model/cuda_backend.py:40-41), so the aux grad reaches only
+            # the router. A plain linear router computes the same logits both
+            # times: one pass serves both (RouterLinearFN keeps the two
+            # gradients apart; without gradients nothing has to).
+            aux_logits = None
+            if plain and torch.is_grad_enabled() and self.router.weight.shape[0] <= 32:
+                logits, aux_logits = router_linear_fn(flat, self.router.weight)
+            else:
+                logits = self.router(flat.to(router_dtype))
+                if plain and not torch.is_grad_enabled():
+                    aux_logits = logits
+        if aux_logits is None:
+            aux_logits = self.router(flat.detach().to(router_dtype))
         out, counts, _ = moe_forward_from_logits(
             flat, logits, self.experts, self.cfg.num_experts, self.cfg.top_k
         )
-        stats = MoELayerStats(tokens_per_expert=counts.detach(), probs_per_expert=aux_probs,
-                              cfg=self.cfg)
+        if plain:
+            stats = MoELayerStats.from_logits(counts.detach(), aux_logits, self.cfg)
+        else:
+            stats = MoELayerStats(tokens_per_expert=counts.detach(),
+                                  probs_per_expert=aux_logits.softmax(dim=-1), cfg=self.cfg)
         return out.reshape(batch, seq_len, d_model), stats
 
 

@@ -407,6 +407,84 @@ class RouteDispatchFN(torch.autograd.Function):
         return dlogits, None, X_grad, None
 
 
+class RouterLinearFN(torch.autograd.Function):
+    """The router's logits for its two uses: the gate path and the statistics path.
+
+    The reference runs the router twice, the second time on detached tokens
+    (src/model/cuda_backend.py:27-41), so that the auxiliary loss reaches only
+    the router's weight. Both passes compute the same logits; here one does,
+    and the backward takes the two gradients apart: dx = dl W (gate path
+    only), dW = (dl + da)^T x. x [T,d], weight [E,d] float32, E <= 32.
+    """
+
+    @staticmethod
+    def forward(ctx, x, weight):
+        logits = torch.nn.functional.linear(x.to(weight.dtype), weight)
+        ctx.save_for_backward(x, weight)
+        ctx.set_materialize_grads(False)
+        return logits, logits.detach()
+
+    @staticmethod
+    def backward(ctx, dl, da):
+        x, weight = ctx.saved_tensors
+        need_dx, need_dW = ctx.needs_input_grad
+        if dl is None and da is None:
+            return None, None
+        if torch.is_grad_enabled():  # differentiated again: composed of torch ops
+            dx = (dl @ weight).to(x.dtype) if need_dx and dl is not None else None
+            g = dl if da is None else da if dl is None else dl + da
+            return dx, g.t() @ x.to(weight.dtype) if need_dW else None
+        return get_hip_extension().router_linear_backward(
+            x.contiguous(), weight.contiguous(), None if dl is None else dl.contiguous(),
+            None if da is None else da.contiguous(), need_dx and dl is not None, need_dW)
+
+
+class RouterStatsFN(torch.autograd.Function):
+    """Load-balancing statistics of the logits (reference src/model/utils.py:77-93).
+
+    Returns (total, frac [E], mean [E], aux): counts.sum(), counts / total,
+    softmax(logits).mean(0) and coef * (frac * mean).sum(); mean and aux carry
+    gradients to the logits.
+    """
+
+    @staticmethod
+    def forward(ctx, logits, counts, coef):
+        logits = logits.contiguous()
+        total, frac, mean, aux = get_hip_extension().router_stats(logits, counts.contiguous(),
+                                                                  coef)
+        ctx.save_for_backward(logits, frac)
+        ctx.coef = coef
+        ctx.mark_non_differentiable(total, frac)
+        ctx.set_materialize_grads(False)
+        return total, frac, mean, aux
+
+    @staticmethod
+    def backward(ctx, _dtotal, _dfrac, dmean, daux):
+        logits, frac = ctx.saved_tensors
+        if dmean is None and daux is None:
+            return None, None, None
+        if torch.is_grad_enabled():  # differentiated again: composed of torch ops
+            v = 0.0
+            if daux is not None:
+                v = v + daux * ctx.coef * frac
+            if dmean is not None:
+                v = v + dmean
+            v = v / logits.shape[0]
+            p = logits.softmax(dim=-1)
+            return p * (v - (p * v).sum(dim=-1, keepdim=True)), None, None
+        return get_hip_extension().router_stats_backward(
+            logits, frac, None if daux is None else daux.contiguous(),
+            None if dmean is None else dmean.contiguous(), ctx.coef), None, None
+
+
+def router_linear_fn(x, weight):
+    return RouterLinearFN.apply(x, weight)
+
+
+def router_stats_fn(logits, counts, coef):
+    return RouterStatsFN.apply(logits, counts, coef)
+
+
 def route_fn(logits, top_k):
     return RouteFN.apply(logits, top_k)
 
