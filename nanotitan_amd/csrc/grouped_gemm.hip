@@ -1440,6 +1440,22 @@ bool gelu_split(int dtype, int64_t red) { return dtype == NT_BF16 && red >= 2048
 // columns), else 128 columns and two workgroups per CU (the 14336 -> 4096
 // down-projection runs 174 us on 256).
 constexpr int64_t kFewRows = 32, kFewRowsSwiGLU = 48;
+// Then up to kMidRows: most experts fit one 128-row tile, and weights past
+// the Infinity Cache come from HBM once, so 128x256 tiles keep two 48 KiB
+// stages in flight (us, before -> 128x256; before: 128x128 tiles, or 256-row
+// ones where the rows of all experts together make enough of them):
+//                        mean rows   64          96          112         128
+//   128, 2048 ->  768  up         89 ->  88   93 ->  91  102 ->  93  127 -> 118
+//                      down       91 ->  86  106 ->  91  112 -> 103  110 -> 122
+//                      SwiGLU    186 -> 161  196 -> 170  210 -> 195  205 -> 213
+//     8, 4096 -> 14336 up        188 -> 172  196 -> 175  200 -> 177  269 -> 227
+//                      down      224 -> 206  235 -> 214  248 -> 219  287 -> 230
+//                      SwiGLU    460 -> 390  467 -> 400  474 -> 409  487 -> 527
+//    16,  512 -> 2048  up         12 ->  14   12 ->  14   12 ->  15
+//                      SwiGLU     27 ->  20   27 ->  20   27 ->  20   27 ->  32
+// (the last layer's weights stay in the cache: only its SwiGLU gains).
+constexpr int64_t kMidRows = 112;
+constexpr int64_t kStreamedBytes = int64_t(256) << 20;
 template <int MODE, int EPI>
 int launch_mfma_auto(int dtype, GemmArgs g, int64_t out_cols, hipStream_t s) {
   const int64_t chunks = g.chunk > 0 ? g.E + g.A / g.chunk : g.E;
@@ -1451,11 +1467,13 @@ int launch_mfma_auto(int dtype, GemmArgs g, int64_t out_cols, hipStream_t s) {
   const int64_t experts = std::min<int64_t>(g.E, g.A);  // that can have rows
   const bool few_rows =
       MODE != kDw && g.A <= (EPI == kEpiSwiGLU ? kFewRowsSwiGLU : kFewRows) * experts;
+  const bool mid_rows = MODE != kDw && g.A <= kMidRows * experts;
   // SwiGLU forward: 256 rows x (128 gate | 128 value) columns, waves 4 x 2,
   // so that each wave holds the gate and value tiles of the same outputs.
   if constexpr (EPI == kEpiSwiGLU) {
     (void)tiles256;
     if (few_rows) return launch_mfma<MODE, EPI, 64, 256, 2, 2, 64, 3>(dtype, g, out_cols, s);
+    if (mid_rows) return launch_mfma<MODE, EPI, 128, 256, 4, 2, 64, 3>(dtype, g, out_cols, s);
     return launch_mfma<MODE, EPI, 256, 256, 4, 2, 64, 2>(dtype, g, out_cols, s);
   } else {
     if constexpr (MODE != kDw && (EPI == kEpiPlain || EPI == kEpiGelu)) {
@@ -1464,6 +1482,8 @@ int launch_mfma_auto(int dtype, GemmArgs g, int64_t out_cols, hipStream_t s) {
           return launch_mfma<MODE, EPI, 64, 256, 2, 2, 64, 3>(dtype, g, out_cols, s);
         return launch_mfma<MODE, EPI, 64, 128, 2, 2, 64, 3>(dtype, g, out_cols, s);
       }
+      if (mid_rows && experts * g.K * g.N * 2 > kStreamedBytes)
+        return launch_mfma<MODE, EPI, 128, 256, 2, 4, 64, 3>(dtype, g, out_cols, s);
     }
     if (tiles256 * 2 >= (int64_t)device_cus(s) * 3) {
       if constexpr (MODE != kDw && (EPI == kEpiPlain || EPI == kEpiDualK)) {
