@@ -106,6 +106,10 @@ def family(name: str) -> str:
         return {"00": "gemm_fwd", "01": "gemm_fwd_gelu", "03": "gemm_fwd", "10": "gemm_dx",
                 "12": "gemm_dx_gelu", "14": "gemm_dx_gelu", "15": "gemm_dx",
                 "20": "gemm_dw"}["".join(m.groups())]
+    m = re.search(r"gg_mfma_tail_kernel<[^,]+, (\d+), (\d+)>", name)
+    if m:
+        return {"00": "gemm_fwd", "10": "gemm_dx", "12": "gemm_dx_gelu", "14": "gemm_dx_gelu",
+                "15": "gemm_dx"}["".join(m.groups())]
     m = re.search(r"gg_generic_kernel<[^,]+, (\d+)>", name)
     if m:
         return {"0": "gemm_fwd", "1": "gemm_dx", "2": "gemm_dw"}[m.group(1)]

@@ -290,7 +290,7 @@ int nt_router_linear_backward(int dtype, const void* x, const float* W, const fl
 /* ------------------------------------------------------------- grouped GEMM */
 
 /* Workspace for nt_grouped_gemm_dw and the paired dW + dX calls with these
- * sizes (the forward and dX GEMMs need none; pass NULL, 0). It holds 256
+ * sizes (the forward and dX GEMMs do with none; see below). It holds 256
  * bytes of tile counters (paired calls), then the fp32 partial sums of
  * experts whose reduction is split (skewed routing): at most 256 MiB plus
  * one K*N*4 slab, and 8 bytes per slab and 256x256 dW tile of arrival
@@ -303,6 +303,19 @@ int nt_router_linear_backward(int dtype, const void* x, const float* W, const fl
  * launched just before it, so every replay of the graph starts them from
  * zero. Calls that overlap in time must not share a workspace. */
 size_t nt_grouped_gemm_workspace_bytes(int dtype, int32_t E, int64_t A, int64_t K, int64_t N);
+
+/* Workspace with which nt_grouped_gemm, nt_grouped_gemm_dx (_gelu, _swiglu)
+ * and nt_grouped_gemm_dx2 (and the dX of the dW + dX calls, where larger than
+ * nt_grouped_gemm_workspace_bytes) may cut the tiles of a nearly empty last
+ * round along the reduction, one piece per idle workgroup, and sum the
+ * pieces in order: 0 where these sizes are never cut, else 32 MiB and 4 KiB.
+ * Smaller or NULL: no tile is cut. The result is the same to float32 rounding
+ * of the sums, and the same bits on every call with such a workspace. Contents
+ * and sharing as for nt_grouped_gemm_workspace_bytes. op: the forward, a
+ * one-part dX (with any epilogue), or the two-part dX. */
+enum { NT_GEMM_FWD = 0, NT_GEMM_DX = 1, NT_GEMM_DX2 = 2 };
+size_t nt_grouped_gemm_tail_workspace_bytes(int dtype, int op, int32_t E, int64_t A, int64_t K,
+                                            int64_t N);
 
 /* out[a,:] = X[a,:] @ W[e] for a in [offsets[e], offsets[e+1]), float32
  * accumulation, cast to dtype. X [A,K], W [E,K,N], out [A,N], offsets [E+1]

@@ -39,6 +39,13 @@ struct GemmArgs {
   // to arrive sums its slabs (fold_split_tile). Null: a reduce pass does.
   unsigned long long* done;
   unsigned long long done_epoch;
+  // Tail split (tail_pieces): fp32 partials, one 128x128 slot per workgroup
+  // that can be resident (tail_slots of them, a multiple of 8; 0: no split),
+  // and one arrival counter per slot, tagged with tail_epoch.
+  int32_t tail_slots;
+  float* tail_partial;
+  unsigned long long* tail_ctr;
+  unsigned long long tail_epoch;
 };
 
 // Epilogues: plain store; forward GELU (out = gelu(h), out2 = gelu'(h), h
@@ -613,6 +620,127 @@ __device__ __forceinline__ void swiglu_bwd(AT dh, AT g, AT v, AT& dg, AT& dv) {
   dv = dh * silu;
 }
 
+// The next of `limit` items from a counter tagged with the launch's epoch:
+// high 40 bits the epoch, low 24 the number of claims so far. A claim is one
+// atomic add. An add that finds a word from before this launch (another
+// epoch: an earlier launch's count, or any other leftover data) installs
+// this launch's epoch with one claim taken, by compare-and-swap; if another
+// workgroup installed it first, the claim is counted again by an add. So the
+// counters need no clearing before a launch, and only the first claims of a
+// launch can take more than one atomic.
+constexpr int kClaimBits = 24;
+__device__ int64_t claim_tagged(unsigned long long* ctr, unsigned long long epoch,
+                                int64_t limit) {
+  constexpr unsigned long long kCount = (1ull << kClaimBits) - 1;
+  unsigned long long v = atomicAdd(ctr, 1ull);
+  while ((v >> kClaimBits) != epoch) {
+    const unsigned long long cur =
+        __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if ((cur >> kClaimBits) == epoch) {
+      v = atomicAdd(ctr, 1ull);
+    } else if (atomicCAS(ctr, cur, (epoch << kClaimBits) | 1ull) == cur) {
+      return limit > 0 ? 0 : -1;
+    }
+  }
+  const int64_t cnt = (int64_t)(v & kCount);
+  return cnt < limit ? cnt : -1;
+}
+
+// Tail split of forward / dX launches. The R tiles of an XCD's last round on
+// `cus` compute units are cut along their nk k-steps into S pieces of at
+// least four, one workgroup each; the last piece of a tile to finish sums the
+// fp32 partials of all, in piece order, and runs the epilogue. S is the one
+// with the shortest round: R S pieces of nk / S k-steps on `cus` units (up to
+// `slots` of them resident), plus base + per S k-steps for the sum.
+__device__ __forceinline__ int tail_pieces(int64_t R, int64_t cus, int64_t slots, int64_t nk,
+                                           int base, int per) {
+  if (R <= 0) return 1;
+  int best = 1;
+  int64_t cost = 840 * nk;  // in 1 / 840 of a k-step; 840 = lcm(1..8)
+  for (int S = 2; S <= 8 && R * S <= slots && 4 * S <= nk; ++S) {
+    const int64_t c = ceil_div(R * S, cus) * nk * (840 / S) + 840 * (base + per * S);
+    if (c < cost) {
+      cost = c;
+      best = S;
+    }
+  }
+  return best;
+}
+
+// One piece's 128x128 tile (4 waves of 64x64) to its slot, then: true in the
+// workgroup that finished the tile last, with every piece's partials summed
+// into acc in piece order. `slot0` is the tile's first slot, `ctr` its
+// counter, s_flag an LDS word. Rows past `rows` are neither stored nor read.
+//
+// The slots are written and read with agent-scope accesses (through the L2s,
+// whichever XCD a workgroup runs on), and a wave's writes are complete once
+// its vmcnt is zero; the counter is touched only after that, behind the
+// workgroup's barrier. Agent-scope fences instead write back and invalidate
+// the whole L2 for every piece: they made the GEMMs around them 1.5 to 3
+// times slower than no split.
+__device__ __forceinline__ bool tail_fold(f32x4_t (&acc)[2][2][4], float* slot0, int piece, int S,
+                                          unsigned long long* ctr, unsigned long long epoch,
+                                          int m0, int rows, int32_t* s_flag) {
+  typedef unsigned long long u64;
+  const int wave = threadIdx.x / kWave, lane = lane_id();
+  auto at = [&](int p, int i, int j, int q) {
+    return reinterpret_cast<u64*>(slot0 + (int64_t)p * (128 * 128)) +
+           ((((wave * 2 + i) * 2 + j) * 4 + q) * 2 * kWave + lane);
+  };
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (m0 + 32 * i + 16 * (q >> 1) >= rows) continue;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        u64 v[2];
+        __builtin_memcpy(v, &acc[i][j][q], sizeof(v));
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          __hip_atomic_store(at(piece, i, j, q) + h * kWave, v[h], __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+      }
+    }
+  wait_vmcnt<0>();
+  __syncthreads();
+  if (threadIdx.x == 0) *s_flag = claim_tagged(ctr, epoch, S) == S - 1 ? 1 : 0;
+  __syncthreads();
+  if (*s_flag == 0) return false;
+  // Sixteen loads in flight per lane and piece (block by block, each waited
+  // for, the sum took longer than a piece's k-steps). Rows past `rows` in a
+  // block read what their slots hold; those outputs are not stored.
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    if (m0 + 32 * i >= rows) continue;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) acc[i][j][q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+    for (int p = 0; p < S; ++p) {
+      u64 v[2][4][2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+          for (int h = 0; h < 2; ++h)
+            v[j][q][h] = __hip_atomic_load(at(p, i, j, q) + h * kWave, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          f32x4_t x;
+          __builtin_memcpy(&x, v[j][q], sizeof(x));
+          acc[i][j][q] += x;
+        }
+    }
+  }
+  return true;
+}
+
 // Tile bookkeeping shared by the launchers: n-tiles, m-tile slots and the
 // grid size (one workgroup per tile).
 template <int MODE>
@@ -631,6 +759,9 @@ int64_t plan_tiles(GemmArgs& g, int64_t out_cols, int BM, int BN) {
 }
 
 }  // namespace
+
+// grouped_gemm.hip. CUs of the device that `s` launches on.
+int device_cus(hipStream_t s);
 
 // staged_gemm.hip: whether the register-staged kernel takes this GEMM, and
 // its launch (epilogue fused).

@@ -25,39 +25,36 @@ namespace {
 
 #include "gelu_table_bf16.inc"
 
-// Operand pointers, strides and valid extents of one output tile, for
-// elements of storage type U (uint16_t: bf16 / fp16; float).
-template <typename U>
-struct TileJobT {
-  const U* pa;  // A operand origin (tile rows, reduction 0)
-  const U* pb;  // B operand origin (tile columns, reduction 0)
+// Operand pointers, strides and valid extents of one output tile (bf16 / fp16).
+struct TileJob {
+  const uint16_t* pa;  // A operand origin (tile rows, reduction 0)
+  const uint16_t* pb;  // B operand origin (tile columns, reduction 0)
   int64_t lda, ldb;
   int64_t rows_valid, cols_valid;  // output rows / columns from the tile origin
   int64_t kred;                    // reduction length
-  U* po;
+  uint16_t* po;
   int64_t ldo;
-  U* po2;          // second output (GELU: gelu'(h); SwiGLU: gate / dvalue)
-  U* po3;          // SwiGLU forward: value output
-  const U* paux;   // GELU backward: gelu'(h); SwiGLU backward: gate
-  const U* paux2;  // SwiGLU backward: value
-  const U* pa2;    // two-part dX: second A operand origin
-  const U* pb2;    // SwiGLU forward: value weights; two-part dX: second W
+  uint16_t* po2;          // second output (GELU: gelu'(h); SwiGLU: gate / dvalue)
+  uint16_t* po3;          // SwiGLU forward: value output
+  const uint16_t* paux;   // GELU backward: gelu'(h); SwiGLU backward: gate
+  const uint16_t* paux2;  // SwiGLU backward: value
+  const uint16_t* pa2;    // two-part dX: second A operand origin
+  const uint16_t* pb2;    // SwiGLU forward: value weights; two-part dX: second W
   int64_t kred1;   // two-part dX: reduction length of the first part
   float* pf;       // dW of a split expert: fp32 partial slab origin (or null)
   const float* pf0;  // split dW: the tile's origin in the expert's first slab
   int32_t nch;       // split dW: the expert's reduction chunks
   int64_t done_idx;  // split dW: the tile's arrival counter
 };
-typedef TileJobT<uint16_t> TileJob;
 
 // Operands and extents of logical output tile `logical` (< mtiles * ntn).
 // For the row-tiled modes s_pref must hold the m-tile prefix of the experts
 // (build_m_prefix) and `mtiles` its total.
 // SwiGLU forward tiles are BN wide in the MFMA (gate and value halves) and
 // BN / 2 wide in the output.
-template <int MODE, int BM, int BN, int EPI = kEpiPlain, typename U = uint16_t>
+template <int MODE, int BM, int BN, int EPI = kEpiPlain>
 __device__ __forceinline__ void setup_job(const GemmArgs& g, const int32_t* s_pref, int64_t mtiles,
-                                          int64_t logical, TileJobT<U>& j) {
+                                          int64_t logical, TileJob& j) {
   j.po2 = nullptr;
   j.po3 = nullptr;
   j.paux = nullptr;
@@ -92,14 +89,14 @@ __device__ __forceinline__ void setup_job(const GemmArgs& g, const int32_t* s_pr
       c1 = c0 + g.chunk < r1 ? c0 + g.chunk : r1;
     }
     j.kred = c1 - c0;
-    j.pa = static_cast<const U*>(g.a) + c0 * g.K + (int64_t)mtl * BM;
+    j.pa = static_cast<const uint16_t*>(g.a) + c0 * g.K + (int64_t)mtl * BM;
     j.lda = g.K;
-    j.pb = static_cast<const U*>(g.b) + c0 * g.N + (int64_t)nt * BN;
+    j.pb = static_cast<const uint16_t*>(g.b) + c0 * g.N + (int64_t)nt * BN;
     j.ldb = g.N;
     j.rows_valid = g.K - (int64_t)mtl * BM;
     j.cols_valid = g.N - (int64_t)nt * BN;
     const int64_t tile_off = (int64_t)mtl * BM * g.N + (int64_t)nt * BN;
-    j.po = static_cast<U*>(g.out) + (int64_t)e * g.K * g.N + tile_off;
+    j.po = static_cast<uint16_t*>(g.out) + (int64_t)e * g.K * g.N + tile_off;
     j.ldo = g.N;
     if (nch >= 2) {
       j.pf = g.partial + (int64_t)(s_split[e] + c) * g.K * g.N + tile_off;
@@ -124,43 +121,63 @@ __device__ __forceinline__ void setup_job(const GemmArgs& g, const int32_t* s_pr
       constexpr int64_t BNO = EPI == kEpiSwiGLU ? BN / 2 : BN;  // output columns per tile
       const int64_t wofs = (int64_t)e * g.K * g.N + (int64_t)nt * BNO;
       const int64_t oofs = row0 * g.N + (int64_t)nt * BNO;
-      j.pa = static_cast<const U*>(g.a) + row0 * g.K;
+      j.pa = static_cast<const uint16_t*>(g.a) + row0 * g.K;
       j.lda = g.K;
-      j.pb = static_cast<const U*>(g.b) + wofs;
+      j.pb = static_cast<const uint16_t*>(g.b) + wofs;
       j.ldb = g.N;
       j.cols_valid = g.N - (int64_t)nt * BNO;
       j.kred = g.K;
-      j.po = static_cast<U*>(g.out) + oofs;
+      j.po = static_cast<uint16_t*>(g.out) + oofs;
       j.ldo = g.N;
-      if (g.out2) j.po2 = static_cast<U*>(g.out2) + oofs;
+      if (g.out2) j.po2 = static_cast<uint16_t*>(g.out2) + oofs;
       if (EPI == kEpiSwiGLU) {
-        j.pb2 = static_cast<const U*>(g.b2) + wofs;
-        j.po3 = static_cast<U*>(g.out3) + oofs;
+        j.pb2 = static_cast<const uint16_t*>(g.b2) + wofs;
+        j.po3 = static_cast<uint16_t*>(g.out3) + oofs;
       }
     } else {  // kDx
       const int64_t oofs = row0 * g.K + (int64_t)nt * BN;
-      j.pa = static_cast<const U*>(g.a) + row0 * g.N;
+      j.pa = static_cast<const uint16_t*>(g.a) + row0 * g.N;
       j.lda = g.N;
-      j.pb = static_cast<const U*>(g.b) + (int64_t)e * g.K * g.N + (int64_t)nt * BN * g.N;
+      j.pb = static_cast<const uint16_t*>(g.b) + (int64_t)e * g.K * g.N + (int64_t)nt * BN * g.N;
       j.ldb = g.N;
       j.cols_valid = g.K - (int64_t)nt * BN;
       j.kred = g.N;
-      j.po = static_cast<U*>(g.out) + oofs;
+      j.po = static_cast<uint16_t*>(g.out) + oofs;
       j.ldo = g.K;
-      if (g.aux) j.paux = static_cast<const U*>(g.aux) + oofs;
+      if (g.aux) j.paux = static_cast<const uint16_t*>(g.aux) + oofs;
       if (EPI == kEpiSwiGLUGrad) {
-        j.paux2 = static_cast<const U*>(g.aux2) + oofs;
-        j.po2 = static_cast<U*>(g.out2) + oofs;
+        j.paux2 = static_cast<const uint16_t*>(g.aux2) + oofs;
+        j.po2 = static_cast<uint16_t*>(g.out2) + oofs;
       }
       if (EPI == kEpiDualK) {
-        j.pa2 = static_cast<const U*>(g.a2) + row0 * g.N;
-        j.pb2 = static_cast<const U*>(g.b2) + (int64_t)e * g.K * g.N +
+        j.pa2 = static_cast<const uint16_t*>(g.a2) + row0 * g.N;
+        j.pb2 = static_cast<const uint16_t*>(g.b2) + (int64_t)e * g.K * g.N +
                 (int64_t)nt * BN * g.N;
         j.kred1 = g.N;
         j.kred = 2 * g.N;
       }
     }
   }
+}
+
+// A tail piece's part of a forward / dX tile (piece -1: the whole tile):
+// k-steps nk piece / np .. nk (piece + 1) / np, as a job of its own.
+template <int MODE, int BK>
+__device__ __forceinline__ void cut_job(TileJob& j, int piece, int np) {
+  if (piece < 0) return;
+  const int64_t nk = ceil_div(j.kred, BK);
+  const int64_t k0 = nk * piece / np * BK, k1 = nk * (piece + 1) / np * BK;
+  const int64_t end = k1 < j.kred ? k1 : j.kred;
+  if (j.kred1 > 0 && k0 >= j.kred1) {  // two-part dX: wholly in the second part
+    j.pa = j.pa2 + (k0 - j.kred1);
+    j.pb = j.pb2 + (k0 - j.kred1);
+    j.kred1 = end - k0;
+  } else {
+    j.pa += k0;
+    j.pb += MODE == kFwd ? k0 * j.ldb : k0;
+    if (j.kred1 > 0) j.kred1 -= k0;
+  }
+  j.kred = end - k0;
 }
 
 // Global loads of one k-step of both operands of a tile into an LDS stage.
@@ -773,32 +790,6 @@ struct GemmLds {
   static constexpr int kTabOff = kTab ? (kGeluTabWords * 4 + 1023) / 1024 * 1024 : 0;
 };
 
-// The next of `limit` items from a counter tagged with the launch's epoch:
-// high 40 bits the epoch, low 24 the number of claims so far. A claim is one
-// atomic add. An add that finds a word from before this launch (another
-// epoch: an earlier launch's count, or any other leftover data) installs
-// this launch's epoch with one claim taken, by compare-and-swap; if another
-// workgroup installed it first, the claim is counted again by an add. So the
-// counters need no clearing before a launch, and only the first claims of a
-// launch can take more than one atomic.
-constexpr int kClaimBits = 24;
-__device__ int64_t claim_tagged(unsigned long long* ctr, unsigned long long epoch,
-                                int64_t limit) {
-  constexpr unsigned long long kCount = (1ull << kClaimBits) - 1;
-  unsigned long long v = atomicAdd(ctr, 1ull);
-  while ((v >> kClaimBits) != epoch) {
-    const unsigned long long cur =
-        __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if ((cur >> kClaimBits) == epoch) {
-      v = atomicAdd(ctr, 1ull);
-    } else if (atomicCAS(ctr, cur, (epoch << kClaimBits) | 1ull) == cur) {
-      return limit > 0 ? 0 : -1;
-    }
-  }
-  const int64_t cnt = (int64_t)(v & kCount);
-  return cnt < limit ? cnt : -1;
-}
-
 // Split dW tile of a paired launch, after its fp32 partial is stored: every
 // wave publishes its stores at agent scope (the slabs are read by a
 // workgroup on any XCD), then one thread counts the chunk on the tile's
@@ -847,12 +838,15 @@ __device__ void fold_split_tile(const GemmArgs& g, const TileJob& j, int64_t* s_
 // The tile loop of workgroup `wg` of `G` that share this GEMM (the kernel's
 // body; gg_pair_kernel runs two of them side by side).
 template <typename T, int MODE, int BM, int BN, int WGM, int WGN, int BK, int NS, int EPI,
-          bool SPLIT, bool DYN = false>
+          bool SPLIT, bool DYN = false, bool TAIL = false>
 __device__ __forceinline__ void gemm_tiles(const GemmArgs& g, int64_t wg, int64_t G, char* smem,
                                            int32_t* s_pref, uint32_t* s_gtab,
                                            unsigned long long* dyn = nullptr,
                                            int64_t* s_next = nullptr,
                                            unsigned long long epoch = 0) {
+  static_assert(!TAIL || (MODE != kDw && !DYN && !SPLIT && BM == 128 && BN == 128 && WGM == 2 &&
+                          WGN == 2),
+                "tail split: forward / dX on 128x128 tiles (tail_fold's slots)");
   constexpr int NW = WGM * WGN;
   constexpr int WM = BM / WGM, WN = BN / WGN;
   constexpr int TM = WM / 32, TN = WN / 32;
@@ -898,9 +892,35 @@ __device__ __forceinline__ void gemm_tiles(const GemmArgs& g, int64_t wg, int64_
   // Row-tiled modes snap the XCD ranges to expert boundaries where they can.
   const int64_t t_end = MODE == kDw ? total * (before + nbx) / G
                                     : xcd_range_start(total, before + nbx, G, s_pref, g.E, g.ntn);
-  int64_t logical = (MODE == kDw ? total * before / G
-                                 : xcd_range_start(total, before, G, s_pref, g.E, g.ntn)) +
-                    wg / kXcd;
+  const int64_t t_beg = MODE == kDw ? total * before / G
+                                    : xcd_range_start(total, before, G, s_pref, g.E, g.ntn);
+  int64_t logical = t_beg + wg / kXcd;
+  // Tail split: tiles from t_full on are np workgroups each; tile_range gives
+  // this workgroup's k-steps of the tile it takes at `t`, and the tile.
+  int64_t t_full = t_end;
+  int np = 1, piece = 0;
+  if constexpr (TAIL) {
+    if (g.tail_slots > 0) {
+      const int64_t red = MODE == kFwd ? g.K : (kDual == 2 ? 2 * g.N : g.N);
+      const int64_t R = (t_end - t_beg) % nbx;
+      // Its k-steps are three times as short as the staged kernel's, so the
+      // sum costs that many more of them.
+      np = tail_pieces(R, nbx, nbx, ceil_div(red, BK), 16, 2);
+      if (np >= 2) t_full = t_end - R;
+      else np = 1;
+    }
+  }
+  // The tile after (or at) logical position t, or -1; sets `piece` (-1: the
+  // whole tile).
+  auto tail_item = [&](int64_t t) -> int64_t {
+    piece = -1;
+    if (t < t_full) return t;
+    if (np < 2 || t >= t_full + nbx) return -1;  // positions t_full .. + nbx: one per workgroup
+    const int64_t r = t - t_full;
+    if (r >= (t_end - t_full) * np) return -1;
+    piece = (int)(r % np);
+    return t_full + r / np;
+  };
   // Dynamic order (DYN): the tiles form kXcd contiguous parts;
   // workgroup wg takes the next tile of its XCD's part from the epoch-tagged
   // counter dyn[p] (claim_tagged), then those of the following parts. One
@@ -921,6 +941,8 @@ __device__ __forceinline__ void gemm_tiles(const GemmArgs& g, int64_t wg, int64_
     const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)((uint64_t)v >> 32));
     return (int64_t)(((uint64_t)hi << 32) | lo);
   };
+  int64_t pos = 0;  // TAIL: this workgroup's position in the order of items
+  (void)pos;
   if constexpr (DYN) {
     if (threadIdx.x == 0) *s_next = claim();
     __syncthreads();
@@ -929,7 +951,15 @@ __device__ __forceinline__ void gemm_tiles(const GemmArgs& g, int64_t wg, int64_
   } else {
     (void)claim;
     (void)uniform;
-    if (logical >= t_end) return;
+    if constexpr (TAIL) {
+      const int64_t t = tail_item(logical);
+      if (t < 0) return;
+      pos = logical;
+      logical = t;
+    } else {
+      (void)tail_item;
+      if (logical >= t_end) return;
+    }
   }
 
   const int lane = lane_id();
@@ -955,6 +985,7 @@ __device__ __forceinline__ void gemm_tiles(const GemmArgs& g, int64_t wg, int64_
   const bool loader = !kSplit || wave < NL;
   TileJob job;
   setup_job<MODE, BM, BN, EPI>(g, s_pref, mtiles, logical, job);
+  if constexpr (TAIL) cut_job<MODE, BK>(job, piece, np);
   Loader ld;
   ld.init(job, wave, lane);
   int64_t nk = ceil_div(job.kred, BK);
@@ -1075,10 +1106,16 @@ __device__ __forceinline__ void gemm_tiles(const GemmArgs& g, int64_t wg, int64_
     }
     __syncthreads();
     if constexpr (DYN) next = uniform(*s_next);
-    const bool more = DYN ? next >= 0 : next < t_end;
+    const int done_piece = piece;  // of the tile just multiplied
+    if constexpr (TAIL) {
+      pos += nbx;
+      next = done_piece >= 0 ? -1 : tail_item(pos);
+    }
+    const bool more = DYN || TAIL ? next >= 0 : next < t_end;
     TileJob nj;
     if (more) {
       setup_job<MODE, BM, BN, EPI>(g, s_pref, mtiles, next, nj);
+      if constexpr (TAIL) cut_job<MODE, BK>(nj, piece, np);
       ld.init(nj, wave, lane);
       nk = ceil_div(nj.kred, BK);
       if (loader) {
@@ -1089,6 +1126,17 @@ __device__ __forceinline__ void gemm_tiles(const GemmArgs& g, int64_t wg, int64_
     }
     static_assert(kLdsEpi || EPI == kEpiPlain, "fused epilogues use the LDS-staged store");
     stores_out = false;
+    if constexpr (TAIL) {
+      // a piece is its workgroup's last item: nothing is in flight past it
+      if (done_piece >= 0) {
+        const int64_t r = wg / kXcd;
+        const int64_t slot0 = xcd * (g.tail_slots / kXcd) + r - done_piece;
+        const int rows = (int)(job.rows_valid < BM ? job.rows_valid : BM);
+        if (!tail_fold(acc, g.tail_partial + slot0 * (BM * BN), done_piece, np, g.tail_ctr + slot0,
+                       g.tail_epoch, wm * WM, rows, reinterpret_cast<int32_t*>(s_next)))
+          return;
+      }
+    }
     if (MODE == kDw && job.pf != nullptr) {
       store_partial(acc, job, wm * WM, wn * WN, lane);
       if (g.done != nullptr) {
@@ -1181,6 +1229,20 @@ gg_mfma_kernel(GemmArgs g) {
   __shared__ int32_t s_pref[L::kPref];
   gemm_tiles<T, MODE, BM, BN, WGM, WGN, BK, NS, EPI, SPLIT>(
       g, blockIdx.x, gridDim.x, lds + L::kTabOff, s_pref, reinterpret_cast<uint32_t*>(lds));
+}
+
+// 128x128 tiles with the tail split, two workgroups per CU (the bound keeps
+// their registers at 256: the fold's loads took them past it).
+template <typename T, int MODE, int EPI>
+__global__ void __launch_bounds__(4 * kWave, 2)
+gg_mfma_tail_kernel(GemmArgs g) {
+  stagger_wait(g.stagger);
+  typedef GemmLds<T, MODE, 128, 128, 2, 2, 64, 2, EPI, false> L;
+  __shared__ __attribute__((aligned(1024))) char lds[L::kSmem];
+  __shared__ int32_t s_pref[L::kPref];
+  __shared__ int64_t s_flag;
+  gemm_tiles<T, MODE, 128, 128, 2, 2, 64, 2, EPI, false, false, true>(
+      g, blockIdx.x, gridDim.x, lds, s_pref, nullptr, nullptr, &s_flag);
 }
 
 // A dW and a dX-type GEMM in one launch, side by side: workgroups [0, nw)
@@ -1325,6 +1387,7 @@ bool mfma_ok(int dtype, int64_t K, int64_t N, const void* p0, const void* p1, co
   return al % 16 == 0;
 }
 
+}  // namespace
 // CUs of the device that `s` launches on (the null stream: the current
 // device). Concurrent first calls may both query; they store the same value.
 int device_cus(hipStream_t s) {
@@ -1340,6 +1403,7 @@ int device_cus(hipStream_t s) {
   }
   return n;
 }
+namespace {
 
 // Workgroups of `kernel` that fit on one CU at once.
 template <typename K>
@@ -1375,7 +1439,8 @@ int32_t stagger_ticks(int mode, int epi, int64_t red, int64_t tiles, int64_t cus
   return (int32_t)(bytes / 60000 * (gelu_many ? 3 : 2) / 2);  // bytes / 6 TB/s, in 10 ns ticks
 }
 
-template <int MODE, int EPI, int BM, int BN, int WGM, int WGN, int BK, int NS, bool SPLIT = false>
+template <int MODE, int EPI, int BM, int BN, int WGM, int WGN, int BK, int NS, bool SPLIT = false,
+          bool TAIL = false>
 int launch_mfma(int dtype, GemmArgs g, int64_t out_cols, hipStream_t s) {
   const int64_t tiles = plan_tiles<MODE>(g, out_cols, BM, EPI == kEpiSwiGLU ? BN / 2 : BN);
   if (tiles == 0) return NT_OK;
@@ -1386,11 +1451,21 @@ int launch_mfma(int dtype, GemmArgs g, int64_t out_cols, hipStream_t s) {
     g.stagger = stagger_ticks(MODE, EPI, red, real_tiles, device_cus(s), BM, BN);
   }
   constexpr int threads = WGM * WGN * kWave;
-  auto kb = gg_mfma_kernel<bf16, MODE, BM, BN, WGM, WGN, BK, NS, EPI, SPLIT>;
+  auto kernel = [](auto t) {
+    typedef decltype(t) T;
+    if constexpr (TAIL) return &gg_mfma_tail_kernel<T, MODE, EPI>;
+    else return &gg_mfma_kernel<T, MODE, BM, BN, WGM, WGN, BK, NS, EPI, SPLIT>;
+  };
+  auto kb = kernel(bf16{});
   // Occupancy of this instantiation (bf16 and fp16 share resource usage).
   static const int per_cu = blocks_per_cu(kb, threads);
   // Persistent: at most one resident wave of workgroups; each walks tiles.
-  const int64_t nblocks = std::min<int64_t>(tiles, (int64_t)device_cus(s) * per_cu);
+  int64_t nblocks = std::min<int64_t>(tiles, (int64_t)device_cus(s) * per_cu);
+  if (!TAIL) g.tail_slots = 0;
+  if (g.tail_slots > 0) {  // every workgroup that can be resident may take a piece
+    nblocks = std::min<int64_t>((int64_t)device_cus(s) * per_cu, g.tail_slots) / 8 * 8;
+    g.tail_slots = (int32_t)nblocks;
+  }
   const dim3 grid((unsigned)nblocks);
   if (dtype == NT_BF16) {
     hipLaunchKernelGGL(kb, grid, dim3(threads), 0, s, g);
@@ -1399,8 +1474,7 @@ int launch_mfma(int dtype, GemmArgs g, int64_t out_cols, hipStream_t s) {
     // of it is built.
     return NT_ERR_DTYPE;
   } else {
-    hipLaunchKernelGGL((gg_mfma_kernel<f16, MODE, BM, BN, WGM, WGN, BK, NS, EPI, SPLIT>), grid,
-                       dim3(threads), 0, s, g);
+    hipLaunchKernelGGL(kernel(f16{}), grid, dim3(threads), 0, s, g);
   }
   return launch_status();
 }
@@ -1485,6 +1559,7 @@ int launch_mfma_auto(int dtype, GemmArgs g, int64_t out_cols, hipStream_t s) {
       if (mid_rows && experts * g.K * g.N * 2 > kStreamedBytes)
         return launch_mfma<MODE, EPI, 128, 256, 2, 4, 64, 3>(dtype, g, out_cols, s);
     }
+    constexpr bool kTail = MODE == kDx || (MODE == kFwd && EPI == kEpiPlain);
     if (tiles256 * 2 >= (int64_t)device_cus(s) * 3) {
       if constexpr (MODE != kDw && (EPI == kEpiPlain || EPI == kEpiDualK)) {
         const int64_t red = MODE == kFwd ? g.K : (EPI == kEpiDualK ? 2 * g.N : g.N);
@@ -1496,6 +1571,10 @@ int launch_mfma_auto(int dtype, GemmArgs g, int64_t out_cols, hipStream_t s) {
           return launch_mfma<MODE, EPI, 256, 256, 2, 4, 64, 2, true>(dtype, g, out_cols, s);
       }
       return launch_mfma<MODE, EPI, 256, 256, 2, 4, 64, 2>(dtype, g, out_cols, s);
+    }
+    if constexpr (kTail) {
+      if (g.tail_slots > 0)
+        return launch_mfma<MODE, EPI, 128, 128, 2, 2, 64, 2, false, true>(dtype, g, out_cols, s);
     }
     return launch_mfma<MODE, EPI, 128, 128, 2, 2, 64, 2>(dtype, g, out_cols, s);
   }
@@ -1811,14 +1890,18 @@ int check_gemm(int dtype, int32_t E, int64_t A, int64_t K, int64_t N, const void
 namespace nt {
 namespace {
 
+int attach_tail(GemmArgs& g, int op, int dtype, void* ws, size_t ws_bytes, hipStream_t stream);
+
 // dX-type GEMM (plain, or with the GELU backward when act_grad is set) and
 // dW; the C entry points below wrap them.
 template <int EPI>
 int dx_impl(int dtype, const void* W, const int32_t* offsets, const void* dOut,
-            const void* act_grad, int32_t E, int64_t A, int64_t K, int64_t N, void* dX,
-            hipStream_t stream) {
+            const void* act_grad, int32_t E, int64_t A, int64_t K, int64_t N, void* dX, void* ws,
+            size_t ws_bytes, hipStream_t stream) {
   if (A == 0 || K == 0) return NT_OK;
   GemmArgs g{dOut, W, offsets, E, A, K, N, dX, 0, 0, 0, nullptr, act_grad, 0, nullptr};
+  const int st = attach_tail(g, NT_GEMM_DX, dtype, ws, ws_bytes, stream);
+  if (st != NT_OK) return st;
   bool mfma = mfma_ok(dtype, K, N, dOut, W, dX);
   if (EPI == kEpiGeluGrad) mfma = mfma && reinterpret_cast<uintptr_t>(act_grad) % 16 == 0;
   return launch_mode<kDx, EPI>(dtype, g, K, mfma, stream);
@@ -1903,6 +1986,67 @@ unsigned long long next_claim_epoch() {
   return e;
 }
 
+// Shapes whose dW and dX share a launch (pair_dw_dx; what else it needs is
+// there). Few experts only: with many (C3: 64, Zipf-skewed) the total work
+// is small next to one 256x256 dW tile over a whole chunk of a heavy expert,
+// which then becomes the critical path (measured: C3 1.37 -> 1.53 ms per
+// layer step paired), while 128x128 tiles balance it.
+bool pair_shape(int32_t E, int64_t K, int64_t N, int64_t cus) {
+  const int64_t dw_tiles = (int64_t)E * ceil_div(K, 256) * ceil_div(N, 256);
+  return E <= kPairMaxExperts && dw_tiles * 2 < cus * 3 &&
+         round_up(dw_tiles, 8) <= cus - cus / 4 && cus % 8 == 0;
+}
+
+// Tail split (tail_pieces): GEMMs whose reduction is longer than their
+// output rows (down projections, and the dX of up projections: few tiles, of
+// many k-steps each) and which are a few rounds of tiles at most. Not the
+// shapes that run paired with their dW: a separate dX is bit-equal to that.
+// A dX is cut the same way with and without a fused activation, whose values
+// stay those of the activation applied to the separate dX.
+// The GEMMs of wide outputs stay whole, so the SwiGLU forward's gate and
+// value are the separate GEMMs' bits there. Measured on MI355X, whole tiles
+// to cut: bf16, two-part dX over 2 x 2048 to 512 for 16 experts: 4,096 rows
+// 49 to 40 us, 32,768 rows 157 to 144; down 14336 -> 4096 for 8 experts,
+// 4,096 rows 727 to 593. fp32, down 2048 -> 512 for 8 experts: 1,040 rows 117
+// to 40 us, 8,192 rows 154 to 121. bf16, down 1365 -> 512 for 8 experts:
+// 1,040 rows 31 to 22 us, 8,192 rows 41 to 34.
+constexpr int32_t kTailSlots = 512;
+constexpr size_t kTailCtrBytes = kTailSlots * 8;
+constexpr size_t kTailBytes = kTailCtrBytes + (size_t)kTailSlots * 128 * 128 * 4;
+size_t tail_bytes(int op, int dtype, int32_t E, int64_t A, int64_t K, int64_t N) {
+  if (dtype_bytes(dtype) == 0 || dtype == NT_F64 || E < 1 || A < 1 || K < 1 || N < 1) return 0;
+  const int64_t red = op == NT_GEMM_FWD ? K : N, out = op == NT_GEMM_FWD ? N : K;
+  if (red <= out || red < 512) return 0;
+  // The aligned 16-bit kernel needs more than 32 k-steps of 64 for a gain: at
+  // 32, 2048 -> 512 for 4,096 rows of 16 experts, the split took 30.8 us, whole
+  // tiles 27.6.
+  if (dtype != NT_F32 && K % 8 == 0 && N % 8 == 0 && red * (op == NT_GEMM_DX2 ? 2 : 1) <= 2048)
+    return 0;
+  if (op != NT_GEMM_FWD && dtype != NT_F32 && K % 8 == 0 && N % 8 == 0 &&
+      pair_shape(E, K, N, kDwSplitCus))
+    return 0;
+  const int64_t tiles = (ceil_div(A, 128) + std::min<int64_t>(E, A)) * ceil_div(out, 128);
+  return tiles <= 4 * 2 * kDwSplitCus ? kTailBytes : 0;
+}
+int attach_tail(GemmArgs& g, int op, int dtype, void* ws, size_t ws_bytes, hipStream_t stream) {
+  const size_t need = tail_bytes(op, dtype, g.E, g.A, g.K, g.N);
+  if (need == 0 || ws == nullptr || ws_bytes < need || reinterpret_cast<uintptr_t>(ws) % 16 != 0)
+    return NT_OK;
+  g.tail_slots = kTailSlots;
+  g.tail_ctr = static_cast<unsigned long long*>(ws);
+  g.tail_partial = reinterpret_cast<float*>(static_cast<char*>(ws) + kTailCtrBytes);
+  g.tail_epoch = next_claim_epoch();
+  // A replayed graph repeats the epoch: clear the counters in the graph (as
+  // the paired launch does).
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusActive) {
+    hipLaunchKernelGGL(zero_u64_kernel, dim3(1), dim3(256), 0, stream, g.tail_ctr,
+                       (int64_t)kTailSlots);
+    return launch_status();
+  }
+  return NT_OK;
+}
+
 template <int EPIX>
 int pair_dw_dx(int dtype, const void* X, const int32_t* offsets, const void* dOut, int32_t E,
                int64_t A, int64_t K, int64_t N, void* dW, void* ws, size_t ws_bytes,
@@ -1918,13 +2062,8 @@ int pair_dw_dx(int dtype, const void* X, const int32_t* offsets, const void* dOu
   // the host's upper bound on chunks would leave workgroups idle.
   const int64_t dw_tiles = (int64_t)E * ceil_div(K, 256) * ceil_div(N, 256);
   const int64_t nw = round_up(dw_tiles, 8);
-  // Few experts only: with many (C3: 64, Zipf-skewed) the total work is
-  // small next to one 256x256 dW tile over a whole chunk of a heavy expert,
-  // which then becomes the critical path (measured: C3 1.37 -> 1.53 ms per
-  // layer step paired), while 128x128 tiles balance it.
   const bool pair = mfma_dw && dx_mfma && A > 0 && K > 0 && N > 0 && aligned &&
-                    ws_bytes >= kCtrBytes && E <= kPairMaxExperts && dw_tiles * 2 < cus * 3 &&
-                    nw <= cus - cus / 4 && cus % 8 == 0 &&
+                    ws_bytes >= kCtrBytes && pair_shape(E, K, N, cus) &&
                     // claim counts stay below 2^kClaimBits: every tile once, plus
                     // at most one failed claim per part per claim call
                     ((ceil_div(A, 256) + E) * ceil_div(K, 256) + 64) * 9 <
@@ -1932,6 +2071,10 @@ int pair_dw_dx(int dtype, const void* X, const int32_t* offsets, const void* dOu
   if (!pair) {
     const int st = dw_impl(dtype, X, offsets, dOut, E, A, K, N, dW, ws, ws_bytes, stream);
     if (st != NT_OK) return st;
+    // the dW and its reduce are done with the workspace (stream order)
+    const int tst = attach_tail(gx, EPIX == kEpiDualK ? NT_GEMM_DX2 : NT_GEMM_DX, dtype, ws,
+                                ws_bytes, stream);
+    if (tst != NT_OK) return tst;
     return launch_mode<kDx, EPIX>(dtype, gx, K, dx_mfma, stream);
   }
   GemmArgs gw{X, dOut, offsets, E, A, K, N, dW, 0, 0, 0, nullptr, nullptr, 0, nullptr};
@@ -2005,15 +2148,21 @@ size_t nt_grouped_gemm_workspace_bytes(int dtype, int32_t E, int64_t A, int64_t 
   return kCtrBytes + dw_ws_bytes(A, K, N, E);
 }
 
+size_t nt_grouped_gemm_tail_workspace_bytes(int dtype, int op, int32_t E, int64_t A, int64_t K,
+                                            int64_t N) {
+  if (op != NT_GEMM_FWD && op != NT_GEMM_DX && op != NT_GEMM_DX2) return 0;
+  return tail_bytes(op, dtype, E, A, K, N);
+}
+
 int nt_grouped_gemm(int dtype, const void* X, const int32_t* offsets, const void* W, int32_t E,
                     int64_t A, int64_t K, int64_t N, void* out, void* ws, size_t ws_bytes,
                     hipStream_t stream) {
-  (void)ws;
-  (void)ws_bytes;
   int st = check_gemm(dtype, E, A, K, N, X, W, offsets, out);
   if (st != NT_OK) return st;
   if (A == 0 || N == 0) return NT_OK;
   GemmArgs g{X, W, offsets, E, A, K, N, out, 0, 0, 0, nullptr, nullptr, 0, nullptr};
+  st = attach_tail(g, NT_GEMM_FWD, dtype, ws, ws_bytes, stream);
+  if (st != NT_OK) return st;
   return launch_mode<kFwd, kEpiPlain>(dtype, g, N, mfma_ok(dtype, K, N, X, W, out), stream);
 }
 
@@ -2035,22 +2184,19 @@ int nt_grouped_gemm_gelu(int dtype, const void* X, const int32_t* offsets, const
 int nt_grouped_gemm_dx(int dtype, const void* W, const int32_t* offsets, const void* dOut,
                        int32_t E, int64_t A, int64_t K, int64_t N, void* dX, void* ws,
                        size_t ws_bytes, hipStream_t stream) {
-  (void)ws;
-  (void)ws_bytes;
   int st = check_gemm(dtype, E, A, K, N, dOut, W, offsets, dX, kDx);
   if (st != NT_OK) return st;
-  return dx_impl<kEpiPlain>(dtype, W, offsets, dOut, nullptr, E, A, K, N, dX, stream);
+  return dx_impl<kEpiPlain>(dtype, W, offsets, dOut, nullptr, E, A, K, N, dX, ws, ws_bytes, stream);
 }
 
 int nt_grouped_gemm_dx_gelu(int dtype, const void* W, const int32_t* offsets, const void* dOut,
                             const void* act_grad, int32_t E, int64_t A, int64_t K, int64_t N,
                             void* dH, void* ws, size_t ws_bytes, hipStream_t stream) {
-  (void)ws;
-  (void)ws_bytes;
   int st = check_gemm(dtype, E, A, K, N, dOut, W, offsets, dH, kDx);
   if (st != NT_OK) return st;
   if (act_grad == nullptr && A > 0 && K > 0) return NT_ERR_INVALID_ARG;
-  return dx_impl<kEpiGeluGrad>(dtype, W, offsets, dOut, act_grad, E, A, K, N, dH, stream);
+  return dx_impl<kEpiGeluGrad>(dtype, W, offsets, dOut, act_grad, E, A, K, N, dH, ws, ws_bytes,
+                               stream);
 }
 
 int nt_grouped_gemm_swiglu(int dtype, const void* X, const int32_t* offsets, const void* W_gate,
@@ -2076,8 +2222,6 @@ int nt_grouped_gemm_dx_swiglu(int dtype, const void* W, const int32_t* offsets, 
                               const void* gate, const void* value, int32_t E, int64_t A,
                               int64_t K, int64_t N, void* dgate, void* dvalue, void* ws,
                               size_t ws_bytes, hipStream_t stream) {
-  (void)ws;
-  (void)ws_bytes;
   int st = check_gemm(dtype, E, A, K, N, dOut, W, offsets, dgate, kDx);
   if (st != NT_OK) return st;
   if (A > 0 && K > 0 && (dvalue == nullptr || gate == nullptr || value == nullptr))
@@ -2085,6 +2229,8 @@ int nt_grouped_gemm_dx_swiglu(int dtype, const void* W, const int32_t* offsets, 
   if (A == 0 || K == 0) return NT_OK;
   GemmArgs g{dOut, W, offsets, E, A, K, N, dgate, 0, 0, 0, dvalue, gate, 0, nullptr,
              nullptr, nullptr, nullptr, value};
+  st = attach_tail(g, NT_GEMM_DX, dtype, ws, ws_bytes, stream);
+  if (st != NT_OK) return st;
   const uintptr_t al = reinterpret_cast<uintptr_t>(dvalue) | reinterpret_cast<uintptr_t>(gate) |
                        reinterpret_cast<uintptr_t>(value);
   const bool mfma = mfma_ok(dtype, K, N, dOut, W, dgate) && al % 16 == 0;
@@ -2094,14 +2240,14 @@ int nt_grouped_gemm_dx_swiglu(int dtype, const void* W, const int32_t* offsets, 
 int nt_grouped_gemm_dx2(int dtype, const void* W1, const void* W2, const int32_t* offsets,
                         const void* dOut1, const void* dOut2, int32_t E, int64_t A, int64_t K,
                         int64_t N, void* dX, void* ws, size_t ws_bytes, hipStream_t stream) {
-  (void)ws;
-  (void)ws_bytes;
   int st = check_gemm(dtype, E, A, K, N, dOut1, W1, offsets, dX, kDx);
   if (st != NT_OK) return st;
   if (A > 0 && N > 0 && K > 0 && (W2 == nullptr || dOut2 == nullptr)) return NT_ERR_INVALID_ARG;
   if (A == 0 || K == 0) return NT_OK;
   GemmArgs g{dOut1, W1, offsets, E, A, K, N, dX, 0, 0, 0, nullptr, nullptr, 0, nullptr,
              dOut2, W2, nullptr, nullptr};
+  st = attach_tail(g, NT_GEMM_DX2, dtype, ws, ws_bytes, stream);
+  if (st != NT_OK) return st;
   // The MFMA path switches operands at a k-step boundary: N a multiple of 64.
   const uintptr_t al = reinterpret_cast<uintptr_t>(W2) | reinterpret_cast<uintptr_t>(dOut2);
   const bool mfma = mfma_ok(dtype, K, N, dOut1, W1, dX) && al % 16 == 0 && N % 64 == 0;

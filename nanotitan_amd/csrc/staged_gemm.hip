@@ -1,5 +1,7 @@
 // Grouped GEMM forward, dX and dW for operands that the direct-to-LDS kernel
 // does not take: fp32, and bf16 / fp16 off 16-byte chunks.
+#include <algorithm>
+
 #include "gemm_common.hpp"
 
 namespace nt {
@@ -291,7 +293,26 @@ gg_staged_kernel(GemmArgs g) {
   }
   const int xcd = blockIdx.x % 8;
   const int64_t t0 = total * xcd / 8, t1 = total * (xcd + 1) / 8;
-  const int64_t logical = t0 + blockIdx.x / 8;
+  int64_t logical = t0 + blockIdx.x / 8;
+  // Tail split: the XCD's last R tiles are np workgroups each.
+  int np = 1, piece = 0;
+  int64_t slot0 = 0;  // the tile's first partial slot
+  if (MODE != kDw && g.tail_slots > 0) {
+    // One workgroup per CU counts as a full round: alone on its CU it runs at
+    // 85-90% of the rate of two or three together.
+    const int64_t red = MODE == kFwd ? g.K : g.N, slots = g.tail_slots / 8, cus = slots / 2;
+    const int64_t R = (t1 - t0) % cus, full = t1 - t0 - R;
+    np = tail_pieces(R, cus, slots, ceil_div(red, BK) * (EPI == kEpiDualK ? 2 : 1), 4, 1);
+    const int64_t r = blockIdx.x / 8 - full;
+    if (np >= 2 && r >= 0) {
+      if (r >= R * np) return;
+      logical = t0 + full + r / np;
+      piece = (int)(r % np);
+      slot0 = xcd * slots + r - piece;
+    } else {
+      np = 1;
+    }
+  }
   if (logical >= t1) return;
 
   const S *pa, *pb, *pa2 = nullptr, *pb2 = nullptr;
@@ -357,6 +378,7 @@ gg_staged_kernel(GemmArgs g) {
   // k-step kt: the first nk1 of (pa, pb), then (two-part dX) of (pa2, pb2).
   const int64_t nk1 = ceil_div(klen, BK);
   const int64_t nk = nk1 + (EPI == kEpiDualK ? ceil_div(klen2, BK) : 0);
+  const int64_t kb = nk * piece / np, ke = nk * (piece + 1) / np;  // this workgroup's k-steps
   auto left_of = [&](int64_t kt) -> int64_t {
     return EPI == kEpiDualK && kt >= nk1 ? klen2 - (kt - nk1) * BK : klen - kt * BK;
   };
@@ -391,8 +413,8 @@ gg_staged_kernel(GemmArgs g) {
   fb[1].init(kHalves ? 64 + wn * 32 : wn * 64 + 32, lane);
   typedef typename mfma_op<M>::vec vec;
 
-  if (nk > 0) fetch(0);
-  for (int64_t kt = 0; kt < nk; ++kt) {
+  if (kb < ke) fetch(kb);
+  for (int64_t kt = kb; kt < ke; ++kt) {
     __syncthreads();  // the stage's readers are done
     const int64_t left = left_of(kt);
     if (left < BK) {
@@ -402,7 +424,7 @@ gg_staged_kernel(GemmArgs g) {
     ta.store(sa, ra);
     tb.store(sb, rb);
     __syncthreads();
-    if (kt + 1 < nk) fetch(kt + 1);
+    if (kt + 1 < ke) fetch(kt + 1);
 #pragma unroll
     for (int ks = 0; ks < BK / 32; ++ks) {
       vec bv[NP][4];
@@ -459,7 +481,7 @@ gg_staged_kernel(GemmArgs g) {
       zero();
       float* fsa = reinterpret_cast<float*>(smem);
       float* fsb = fsa + BT * TA::kPitch;
-      for (int64_t kt = 0; kt < nk; ++kt) {
+      for (int64_t kt = kb; kt < ke; ++kt) {
         fetch(kt);
         const int64_t left = left_of(kt);
         if (left < BK) {
@@ -486,6 +508,13 @@ gg_staged_kernel(GemmArgs g) {
         }
       }
     }
+  }
+
+  if (MODE != kDw && np > 1) {
+    __shared__ int32_t s_last;
+    if (!tail_fold(acc, g.tail_partial + slot0 * (BT * BT), piece, np, g.tail_ctr + slot0,
+                   g.tail_epoch, wm * 64, rvi, &s_last))
+      return;
   }
 
   S* po = static_cast<S*>(g.out) + oofs;
@@ -551,6 +580,11 @@ int launch_staged(int dtype, GemmArgs g, int64_t out_cols, hipStream_t s) {
   g.chunk = 0;
   int64_t tiles = plan_tiles<MODE>(g, out_cols, BT, EPI == kEpiSwiGLU ? BT / 2 : BT);
   if (tiles == 0) return NT_OK;
+  if (MODE == kDw) g.tail_slots = 0;
+  if (g.tail_slots > 0) {
+    g.tail_slots = std::min<int32_t>(g.tail_slots / 16, device_cus(s) / 8) * 16;  // two per CU
+    tiles += g.tail_slots;
+  }
   tiles = round_up(tiles, 8);
   if (tiles > INT32_MAX) return NT_ERR_TOO_LARGE;
   const dim3 grid((unsigned)tiles), block(kStagedThreads);

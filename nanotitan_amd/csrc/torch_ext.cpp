@@ -76,6 +76,22 @@ Tensor workspace(const Tensor& like, size_t bytes) {
   return at::empty({(int64_t)std::max<size_t>(bytes, 1)}, like.options().dtype(at::kByte));
 }
 
+// Workspace of a forward / dX GEMM whose last round of tiles may be cut into
+// pieces (ws stays undefined where these sizes never are); returns its bytes.
+size_t tail_workspace(const Tensor& like, int op, int32_t E, int64_t A, int64_t K, int64_t N,
+                      Tensor& ws) {
+  const size_t bytes = nt_grouped_gemm_tail_workspace_bytes(dtype_code(like), op, E, A, K, N);
+  if (bytes > 0) ws = workspace(like, bytes);
+  return bytes;
+}
+
+// Of a dW + dX call: the larger of the dW's and its dX's.
+Tensor pair_workspace(const Tensor& like, int op, int32_t E, int64_t A, int64_t K, int64_t N) {
+  const int dt = dtype_code(like);
+  return workspace(like, std::max(nt_grouped_gemm_workspace_bytes(dt, E, A, K, N),
+                                  nt_grouped_gemm_tail_workspace_bytes(dt, op, E, A, K, N)));
+}
+
 // ------------------------------------------------------ reference surface
 
 // count_expert_kernel(topk_experts_per_token, mask, num_experts, num_topk_experts)
@@ -245,9 +261,10 @@ Tensor grouped_gemm_kernel(Tensor X, Tensor offsets, Tensor W) {
   c10::hip::HIPGuard guard(X.get_device());
   Tensor out = at::empty({A, N}, X.options());
   const int dt = dtype_code(X);
-  // The forward and dX GEMMs need no workspace (only the dW split does).
+  Tensor ws;
+  const size_t wb = tail_workspace(X, NT_GEMM_FWD, E, A, K, N, ws);
   check_status(nt_grouped_gemm(dt, X.data_ptr(), offsets.data_ptr<int32_t>(), W.data_ptr(), E, A,
-                               K, N, out.data_ptr(), nullptr, 0, stream_of(X)),
+                               K, N, out.data_ptr(), wb ? ws.data_ptr() : nullptr, wb, stream_of(X)),
                "grouped_gemm_kernel");
   return out;
 }
@@ -283,8 +300,11 @@ Tensor bwd_grouped_gemm_dX_kernel(Tensor W, Tensor offsets, Tensor dOut) {
   c10::hip::HIPGuard guard(W.get_device());
   Tensor dX = at::empty({A, K}, W.options());
   const int dt = dtype_code(W);
+  Tensor ws;
+  const size_t wb = tail_workspace(W, NT_GEMM_DX, E, A, K, N, ws);
   check_status(nt_grouped_gemm_dx(dt, W.data_ptr(), offsets.data_ptr<int32_t>(), dOut.data_ptr(),
-                                  E, A, K, N, dX.data_ptr(), nullptr, 0, stream_of(W)),
+                                  E, A, K, N, dX.data_ptr(), wb ? ws.data_ptr() : nullptr, wb,
+                                  stream_of(W)),
                "bwd_grouped_gemm_dX_kernel");
   return dX;
 }
@@ -327,9 +347,12 @@ Tensor bwd_grouped_gemm_dX_gelu(Tensor W, Tensor offsets, Tensor dOut, Tensor ac
   c10::hip::HIPGuard guard(W.get_device());
   Tensor dH = at::empty({A, K}, W.options());
   const int dt = dtype_code(W);
+  Tensor ws;
+  const size_t wb = tail_workspace(W, NT_GEMM_DX, E, A, K, N, ws);
   check_status(nt_grouped_gemm_dx_gelu(dt, W.data_ptr(), offsets.data_ptr<int32_t>(),
                                        dOut.data_ptr(), act_grad.data_ptr(), E, A, K, N,
-                                       dH.data_ptr(), nullptr, 0, stream_of(W)),
+                                       dH.data_ptr(), wb ? ws.data_ptr() : nullptr, wb,
+                                       stream_of(W)),
                "bwd_grouped_gemm_dX_gelu");
   return dH;
 }
@@ -350,7 +373,7 @@ std::tuple<Tensor, Tensor> bwd_grouped_gemm_dW_dX(Tensor X, Tensor W, Tensor off
   Tensor dW = at::empty({E, K, N}, X.options());
   Tensor dX = at::empty({A, K}, X.options());
   const int dt = dtype_code(X);
-  Tensor ws = workspace(X, nt_grouped_gemm_workspace_bytes(dt, E, A, K, N));
+  Tensor ws = pair_workspace(X, NT_GEMM_DX, E, A, K, N);
   check_status(nt_grouped_gemm_dw_dx(dt, X.data_ptr(), W.data_ptr(), offsets.data_ptr<int32_t>(),
                                      dOut.data_ptr(), E, A, K, N, dW.data_ptr(), dX.data_ptr(),
                                      ws.data_ptr(), ws.numel(), stream_of(X)),
@@ -379,7 +402,7 @@ std::tuple<Tensor, Tensor> bwd_grouped_gemm_dW_dX_gelu(Tensor act, Tensor W, Ten
   Tensor dW = at::empty({E, K, N}, act.options());
   Tensor dH = at::empty({A, K}, act.options());
   const int dt = dtype_code(act);
-  Tensor ws = workspace(act, nt_grouped_gemm_workspace_bytes(dt, E, A, K, N));
+  Tensor ws = pair_workspace(act, NT_GEMM_DX, E, A, K, N);
   check_status(nt_grouped_gemm_dw_dx_gelu(dt, act.data_ptr(), W.data_ptr(),
                                           offsets.data_ptr<int32_t>(), dOut.data_ptr(),
                                           act_grad.data_ptr(), E, A, K, N, dW.data_ptr(),
@@ -414,7 +437,7 @@ std::tuple<Tensor, Tensor, Tensor> bwd_grouped_gemm_dW_dX_swiglu(Tensor hidden, 
   Tensor dgate = at::empty({A, K}, hidden.options());
   Tensor dvalue = at::empty({A, K}, hidden.options());
   const int dt = dtype_code(hidden);
-  Tensor ws = workspace(hidden, nt_grouped_gemm_workspace_bytes(dt, E, A, K, N));
+  Tensor ws = pair_workspace(hidden, NT_GEMM_DX, E, A, K, N);
   check_status(nt_grouped_gemm_dw_dx_swiglu(dt, hidden.data_ptr(), W.data_ptr(),
                                             offsets.data_ptr<int32_t>(), dOut.data_ptr(),
                                             gate.data_ptr(), value.data_ptr(), E, A, K, N,
@@ -442,7 +465,7 @@ std::tuple<Tensor, Tensor> bwd_grouped_gemm_dW_dX2(Tensor X, Tensor W1, Tensor W
   Tensor dW1 = at::empty({E, K, N}, X.options());
   Tensor dX = at::empty({A, K}, X.options());
   const int dt = dtype_code(X);
-  Tensor ws = workspace(X, nt_grouped_gemm_workspace_bytes(dt, E, A, K, N));
+  Tensor ws = pair_workspace(X, NT_GEMM_DX2, E, A, K, N);
   check_status(nt_grouped_gemm_dw_dx2(dt, X.data_ptr(), W1.data_ptr(), W2.data_ptr(),
                                       offsets.data_ptr<int32_t>(), dOut1.data_ptr(),
                                       dOut2.data_ptr(), E, A, K, N, dW1.data_ptr(), dX.data_ptr(),
@@ -498,10 +521,12 @@ std::tuple<Tensor, Tensor> bwd_grouped_gemm_dX_swiglu(Tensor W, Tensor offsets, 
   c10::hip::HIPGuard guard(W.get_device());
   Tensor dgate = at::empty({A, K}, W.options());
   Tensor dvalue = at::empty({A, K}, W.options());
+  Tensor ws;
+  const size_t wb = tail_workspace(W, NT_GEMM_DX, E, A, K, N, ws);
   check_status(nt_grouped_gemm_dx_swiglu(dtype_code(W), W.data_ptr(), offsets.data_ptr<int32_t>(),
                                          dOut.data_ptr(), gate.data_ptr(), value.data_ptr(), E, A,
-                                         K, N, dgate.data_ptr(), dvalue.data_ptr(), nullptr, 0,
-                                         stream_of(W)),
+                                         K, N, dgate.data_ptr(), dvalue.data_ptr(),
+                                         wb ? ws.data_ptr() : nullptr, wb, stream_of(W)),
                "bwd_grouped_gemm_dX_swiglu");
   return {dgate, dvalue};
 }
@@ -519,9 +544,12 @@ Tensor bwd_grouped_gemm_dX2(Tensor W1, Tensor W2, Tensor offsets, Tensor dOut1, 
   const int32_t E = (int32_t)W1.size(0);
   c10::hip::HIPGuard guard(W1.get_device());
   Tensor dX = at::empty({A, K}, W1.options());
+  Tensor ws;
+  const size_t wb = tail_workspace(W1, NT_GEMM_DX2, E, A, K, N, ws);
   check_status(nt_grouped_gemm_dx2(dtype_code(W1), W1.data_ptr(), W2.data_ptr(),
                                    offsets.data_ptr<int32_t>(), dOut1.data_ptr(), dOut2.data_ptr(),
-                                   E, A, K, N, dX.data_ptr(), nullptr, 0, stream_of(W1)),
+                                   E, A, K, N, dX.data_ptr(), wb ? ws.data_ptr() : nullptr, wb,
+                                   stream_of(W1)),
                "bwd_grouped_gemm_dX2");
   return dX;
 }

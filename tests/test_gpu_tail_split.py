@@ -1,0 +1,95 @@
+"""GPU: forward / dX GEMMs whose last round of tiles is cut along the reduction
+(one piece per idle workgroup, partials summed in piece order): against
+float64, run to run, against a call without a workspace, and under graph
+replay with eager calls in between.
+
+Bound as for the uncut GEMM, the order of a sum does not enter it:
+(R + 8) 2^-24 sum |a||b|, then one rounding to p significant bits (2^-p of the
+value; 2^-25 at fp16's subnormals)."""
+
+import pytest
+import torch
+
+from nanotitan_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+HALF_ULP = {torch.bfloat16: 2.0**-8, torch.float16: 2.0**-11, torch.float32: 2.0**-24}
+COUNTS = [200, 0, 129, 128, 300, 1, 0, 255, 77, 256, 90, 131, 140, 127, 2, 260, 130]  # mean 131
+
+
+def _check(out, ref, mag, R, dtype):
+    acc = (R + 8) * 2.0**-24 * mag
+    bound = acc + HALF_ULP[dtype] * (ref.abs() + acc) + 2.0**-25
+    assert bool(((out.cpu().double() - ref).abs() <= bound).all())
+
+
+def _case(dtype, K, N, counts=COUNTS, seed=0):
+    g = torch.Generator().manual_seed(seed + K + N)
+    offs = torch.tensor([0, *torch.tensor(counts).cumsum(0).tolist()], dtype=torch.int32)
+    A, E = sum(counts), len(counts)
+    X = torch.randn(A, K, generator=g).to(dtype)
+    W = torch.randn(E, K, N, generator=g).to(dtype)
+    return offs, X, W, [(e, slice(int(offs[e]), int(offs[e + 1]))) for e in range(E)]
+
+
+@pytest.mark.parametrize("dtype,K,N", [
+    (torch.bfloat16, 4096, 64), (torch.float16, 4104, 264), (torch.bfloat16, 2056, 136),
+    (torch.float32, 512, 130), (torch.float32, 1001, 64), (torch.bfloat16, 1365, 300)])
+def test_tail_pieces(ext, dtype, K, N):
+    offs, X, W, seg = _case(dtype, K, N)
+    A, E = X.shape[0], W.shape[0]
+    code = capi.dtype_code(dtype)
+    assert capi.load().nt_grouped_gemm_tail_workspace_bytes(code, 0, E, A, K, N) > 0
+    assert capi.load().nt_grouped_gemm_tail_workspace_bytes(code, 1, E, A, N, K) > 0
+    og, Xg, Wg = offs.cuda(), X.cuda(), W.cuda()
+
+    def rows(a, b):
+        return torch.cat([a[s].double() @ b[e].double() for e, s in seg])
+
+    ref, mag = rows(X, W), rows(X.abs(), W.abs())
+    out = ext.grouped_gemm_kernel(Xg, og, Wg)
+    _check(out, ref, mag, K, dtype)
+    assert torch.equal(out, ext.grouped_gemm_kernel(Xg, og, Wg))
+    # without a workspace: whole tiles
+    whole = torch.empty_like(out)
+    capi.call("nt_grouped_gemm", code, capi.ptr(Xg), capi.ptr(og), capi.ptr(Wg), E, A, K, N,
+              capi.ptr(whole), None, 0, capi.current_stream())
+    _check(whole, ref, mag, K, dtype)
+    # dX of an up projection N -> K, one and two parts, alone and beside its dW
+    Wt = W.transpose(1, 2).contiguous().cuda()  # [E, N, K]: dX = X @ Wt^T, N columns
+    dX = ext.bwd_grouped_gemm_dX_kernel(Wt, og, Xg)
+    _check(dX, ref, mag, K, dtype)
+    H = torch.randn(A, N, generator=torch.Generator().manual_seed(1)).to(dtype).cuda()
+    assert torch.equal(ext.bwd_grouped_gemm_dW_dX(H, Wt, og, Xg)[1], dX)
+    G, V = (torch.randn(A, N, generator=torch.Generator().manual_seed(s)).to(dtype).cuda()
+            for s in (2, 3))
+    dH = ext.bwd_grouped_gemm_dX_gelu(Wt, og, Xg, H)
+    assert torch.equal(dH, (dX.float() * H.float()).to(dtype))
+    assert torch.equal(ext.bwd_grouped_gemm_dW_dX_gelu(H, Wt, og, Xg, H)[1], dH)
+    dS = ext.bwd_grouped_gemm_dX_swiglu(Wt, og, Xg, G, V)
+    for a, b in zip(ext.bwd_grouped_gemm_dW_dX_swiglu(H, Wt, og, Xg, G, V)[1:], dS):
+        assert torch.equal(a, b)
+    dX2 = ext.bwd_grouped_gemm_dX2(Wt, Wt, og, Xg, Xg)
+    _check(dX2, 2 * ref, 2 * mag, 2 * K, dtype)
+    assert torch.equal(ext.bwd_grouped_gemm_dW_dX2(H, Wt, Wt, og, Xg, Xg)[1], dX2)
+
+
+@pytest.mark.parametrize("dtype,K,N", [(torch.bfloat16, 4096, 128), (torch.float32, 777, 130)])
+def test_tail_pieces_under_graph_replay(ext, dtype, K, N):
+    offs, X, W, _ = _case(dtype, K, N)
+    og, Xg, Wg = offs.cuda(), X.cuda(), W.cuda()
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        ext.grouped_gemm_kernel(Xg, og, Wg)
+    torch.cuda.current_stream().wait_stream(s)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ext.grouped_gemm_kernel(Xg, og, Wg)
+    for seed in range(4):
+        Xg.copy_(_case(dtype, K, N, seed=10 * seed)[1])
+        graph.replay()
+        eager = ext.grouped_gemm_kernel(Xg, og, Wg)
+        torch.cuda.synchronize()
+        assert torch.equal(out, eager), seed
