@@ -33,7 +33,8 @@ from nanotitan_amd.moe_ops import (
     grouped_gelu_ffn_fn,
     route_dispatch_fn,
     route_fn,
-    router_linear_fn,
+    router_aux_fn,
+    router_gate_fn,
     router_stats_fn,
     swiglu_ffn_fn,
 )
@@ -78,15 +79,20 @@ class MoELayerStats:
         )
 
     @classmethod
-    def from_logits(cls, tokens_per_expert, logits, cfg):
-        """The same statistics from the float32 router logits, in one kernel."""
+    def from_logits(cls, tokens_per_expert, logits, cfg, router=None):
+        """The same statistics from the float32 router logits, in one kernel.
+
+        ``router``: (tokens, weight) where the gradient goes to the weight of
+        the linear that gives these logits; else it goes to ``logits``.
+        """
         stats = cls.__new__(cls)
         stats.tokens_per_expert = tokens_per_expert
         stats.cfg = cfg
         stats.num_tokens = logits.shape[0]
+        coef = cfg.router_alpha * cfg.num_experts
         (stats.total_assignments, stats.ass_frac_per_expert, stats.probs_per_expert,
-         stats.aux_loss) = router_stats_fn(logits, tokens_per_expert,
-                                           cfg.router_alpha * cfg.num_experts)
+         stats.aux_loss) = (router_stats_fn(logits, tokens_per_expert, coef) if router is None
+                            else router_aux_fn(logits, *router, tokens_per_expert, coef))
         return stats
 
 
@@ -198,25 +204,28 @@ class HIPMoEBackend:
         plain = (_plain_router(self.router, flat)
                  and type(self.cfg.router_alpha * self.cfg.num_experts) in (int, float))
         with record_function("moe/router"):
-            # Aux-loss logits from a second router pass on detached tokens
+            # Aux-loss logits come from a second router pass on detached tokens
             # (src/model/cuda_backend.py:40-41), so the aux grad reaches only
             # the router. A plain linear router computes the same logits both
-            # times: one pass serves both (RouterLinearFN keeps the two
-            # gradients apart; without gradients nothing has to).
-            aux_logits = None
-            if plain and torch.is_grad_enabled() and self.router.weight.shape[0] <= 32:
-                logits, aux_logits = router_linear_fn(flat, self.router.weight)
+            # times: the second pass is then only its gradient (RouterAuxFN),
+            # and nothing at all without gradients.
+            grad = torch.is_grad_enabled()
+            one_pass = plain and (not grad or self.router.weight.shape[0] <= 32)
+            if one_pass and grad:
+                logits = router_gate_fn(flat, self.router.weight)
             else:
                 logits = self.router(flat.to(router_dtype))
-                if plain and not torch.is_grad_enabled():
-                    aux_logits = logits
-        if aux_logits is None:
+        if one_pass:
+            aux_logits = logits
+        else:
             aux_logits = self.router(flat.detach().to(router_dtype))
         out, counts, _ = moe_forward_from_logits(
             flat, logits, self.experts, self.cfg.num_experts, self.cfg.top_k
         )
         if plain:
-            stats = MoELayerStats.from_logits(counts.detach(), aux_logits, self.cfg)
+            stats = MoELayerStats.from_logits(
+                counts.detach(), aux_logits, self.cfg,
+                router=(flat, self.router.weight) if one_pass and grad else None)
         else:
             stats = MoELayerStats(tokens_per_expert=counts.detach(),
                                   probs_per_expert=aux_logits.softmax(dim=-1), cfg=self.cfg)

@@ -407,36 +407,30 @@ class RouteDispatchFN(torch.autograd.Function):
         return dlogits, None, X_grad, None
 
 
-class RouterLinearFN(torch.autograd.Function):
-    """The router's logits for its two uses: the gate path and the statistics path.
+class RouterGateFN(torch.autograd.Function):
+    """The router's logits x @ weight.T (float32) for the gate path.
 
-    The reference runs the router twice, the second time on detached tokens
-    (src/model/cuda_backend.py:27-41), so that the auxiliary loss reaches only
-    the router's weight. Both passes compute the same logits; here one does,
-    and the backward takes the two gradients apart: dx = dl W (gate path
-    only), dW = (dl + da)^T x. x [T,d], weight [E,d] float32, E <= 32.
+    x [T,d], weight [E,d] float32, E <= 32. One kernel gives dx = dl W and
+    dW = dl^T x (reference src/model/cuda_backend.py:27-30).
     """
 
     @staticmethod
     def forward(ctx, x, weight):
-        logits = torch.nn.functional.linear(x.to(weight.dtype), weight)
         ctx.save_for_backward(x, weight)
         ctx.set_materialize_grads(False)
-        return logits, logits.detach()
+        return torch.nn.functional.linear(x.to(weight.dtype), weight)
 
     @staticmethod
-    def backward(ctx, dl, da):
+    def backward(ctx, dl):
         x, weight = ctx.saved_tensors
         need_dx, need_dW = ctx.needs_input_grad
-        if dl is None and da is None:
+        if dl is None:
             return None, None
         if torch.is_grad_enabled():  # differentiated again: composed of torch ops
-            dx = (dl @ weight).to(x.dtype) if need_dx and dl is not None else None
-            g = dl if da is None else da if dl is None else dl + da
-            return dx, g.t() @ x.to(weight.dtype) if need_dW else None
+            return ((dl @ weight).to(x.dtype) if need_dx else None,
+                    dl.t() @ x.to(weight.dtype) if need_dW else None)
         return get_hip_extension().router_linear_backward(
-            x.contiguous(), weight.contiguous(), None if dl is None else dl.contiguous(),
-            None if da is None else da.contiguous(), need_dx and dl is not None, need_dW)
+            x.contiguous(), weight.contiguous(), dl.contiguous(), None, need_dx, need_dW)
 
 
 class RouterStatsFN(torch.autograd.Function):
@@ -464,21 +458,69 @@ class RouterStatsFN(torch.autograd.Function):
         if dmean is None and daux is None:
             return None, None, None
         if torch.is_grad_enabled():  # differentiated again: composed of torch ops
-            v = 0.0
-            if daux is not None:
-                v = v + daux * ctx.coef * frac
-            if dmean is not None:
-                v = v + dmean
-            v = v / logits.shape[0]
-            p = logits.softmax(dim=-1)
-            return p * (v - (p * v).sum(dim=-1, keepdim=True)), None, None
+            return _stats_dlogits(logits, frac, daux, dmean, ctx.coef), None, None
         return get_hip_extension().router_stats_backward(
             logits, frac, None if daux is None else daux.contiguous(),
             None if dmean is None else dmean.contiguous(), ctx.coef), None, None
 
 
-def router_linear_fn(x, weight):
-    return RouterLinearFN.apply(x, weight)
+def _stats_dlogits(logits, frac, daux, dmean, coef):
+    v = 0.0
+    if daux is not None:
+        v = v + daux * coef * frac
+    if dmean is not None:
+        v = v + dmean
+    v = v / logits.shape[0]
+    p = logits.softmax(dim=-1)
+    return p * (v - (p * v).sum(dim=-1, keepdim=True))
+
+
+class RouterAuxFN(torch.autograd.Function):
+    """RouterStatsFN on the router's second pass, with the gradient to its weight.
+
+    The reference runs the router twice, the second time on detached tokens
+    (src/model/cuda_backend.py:40-41), so that the auxiliary loss reaches only
+    the router's weight. Both passes compute the same logits, so the first
+    pass's are taken; the graph is the second pass's own (one of the two can
+    be differentiated and freed before the other). logits [T,E] float32 =
+    x @ weight.T, x [T,d] and logits without gradients, E <= 32.
+    """
+
+    @staticmethod
+    def forward(ctx, logits, x, weight, counts, coef):
+        logits = logits.contiguous()
+        total, frac, mean, aux = get_hip_extension().router_stats(logits, counts.contiguous(),
+                                                                  coef)
+        ctx.save_for_backward(logits, frac, x, weight)
+        ctx.coef = coef
+        ctx.mark_non_differentiable(total, frac)
+        ctx.set_materialize_grads(False)
+        return total, frac, mean, aux
+
+    @staticmethod
+    def backward(ctx, _dtotal, _dfrac, dmean, daux):
+        logits, frac, x, weight = ctx.saved_tensors
+        if dmean is None and daux is None:
+            return None, None, None, None, None
+        if torch.is_grad_enabled():  # differentiated again: composed of torch ops
+            x = x.to(weight.dtype)
+            da = _stats_dlogits(x @ weight.t(), frac, daux, dmean, ctx.coef)
+            return None, None, da.t() @ x, None, None
+        ext = get_hip_extension()
+        da = ext.router_stats_backward(logits, frac, None if daux is None else daux.contiguous(),
+                                       None if dmean is None else dmean.contiguous(), ctx.coef)
+        _, dW = ext.router_linear_backward(x.contiguous(), weight.contiguous(), None, da, False,
+                                           True)
+        return None, None, dW, None, None
+
+
+def router_gate_fn(x, weight):
+    return RouterGateFN.apply(x, weight)
+
+
+def router_aux_fn(logits, x, weight, counts, coef):
+    """Statistics of RouterStatsFN; logits and x are used without their gradients."""
+    return RouterAuxFN.apply(logits.detach(), x.detach(), weight, counts, coef)
 
 
 def router_stats_fn(logits, counts, coef):

@@ -112,3 +112,39 @@ def test_single_router_pass_matches_two_passes(ext, E):
         for u, v in zip(a, b):
             assert u.dtype == v.dtype and u.shape == v.shape
             torch.testing.assert_close(u, v, rtol=2e-5, atol=2e-6)
+
+
+def _moe(E, dtype=torch.float32, d=48):
+    from nanotitan_amd.layer import MoE
+
+    cfg = SimpleNamespace(d_model=d, num_experts=E, top_k=2, ffn_in=64, dtype=dtype,
+                          moe_router_dtype=torch.float32, moe_backend="hip", router_alpha=0.01)
+    torch.manual_seed(4)
+    moe = MoE(cfg).cuda()
+    for p in moe.experts.parameters():
+        p.data.normal_(0, 0.1)
+    return moe, torch.randn(2, 37, d, device="cuda").to(dtype)
+
+
+@pytest.mark.parametrize("E", [8, 40])  # one pass / two passes in training
+def test_loss_and_output_have_graphs_of_their_own(ext, E):
+    moe, x = _moe(E)
+    params = list(moe.parameters())
+    y, st = moe(x.requires_grad_())
+    together = torch.autograd.grad([y.square().sum() + st.aux_loss], [x, *params])
+    for first in ("loss", "output"):
+        y, st = moe(x)
+        parts = [st.aux_loss, y.square().sum()]
+        for p in (x, *params):
+            p.grad = None
+        for part in parts if first == "loss" else parts[::-1]:
+            part.backward()  # without retain_graph
+        for p, g in zip((x, *params), together):
+            torch.testing.assert_close(p.grad, g, rtol=2e-5, atol=2e-6)
+    # the loss reaches the router's weight alone
+    _, st = moe(x)
+    assert torch.autograd.grad(st.aux_loss, x, allow_unused=True, retain_graph=True)[0] is None
+    moe.router.weight.requires_grad_(False)
+    y, st = moe(x)
+    assert y.requires_grad and not st.aux_loss.requires_grad
+    assert not st.probs_per_expert.requires_grad
