@@ -540,8 +540,8 @@ def cpu_baseline(wl_cpu, budget_s: float = 20.0, warmup: int = 1, max_iters: int
 def profile_fields(wl, ffn_kind):
     """HBM traffic and MFMA busy fraction of the GEMMs from the committed
     rocprofv3 counter summaries (profiles/*.json, written by bench_profiles.py),
-    tagged with the commit whose kernels they were measured on and marked
-    stale when the kernel sources have changed since."""
+    tagged with the commit the measured tree stood on and marked stale when
+    the kernel sources have changed since."""
     out = {}
     if ffn_kind != "gelu":
         return out
@@ -582,7 +582,7 @@ def source_note(path, js):
     """Where a profile figure comes from, and whether the kernel sources it
     was measured on are the ones this run executes."""
     same = js.get("source_hash") == kernel_source_hash(ROOT)
-    return (f"profiles/{path.name}, kernels of commit {js.get('commit', 'unrecorded')}"
+    return (f"profiles/{path.name}, tree on commit {js.get('commit', 'unrecorded')}"
             f"{'' if same else ' (kernel sources changed since: stale)'}")
 
 

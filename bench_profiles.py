@@ -13,7 +13,8 @@ fraction to its JSON line from the summaries this script writes:
 - ``profiles/moe_layer_c<N>_kernel_trace.md`` from a ``--kernel-trace --stats``
   pass, with the bench line that run printed.
 
-Every JSON records the commit it was measured on and ``source_hash``, a hash of
+Every JSON records the commit the measured tree stood on (the parent, where a
+kernel change and its profiles are one commit) and ``source_hash``, a hash of
 the kernel sources (``kernel_source_hash``); ``bench.py`` recomputes the hash
 and reports whether the profile still matches the code it runs.
 
@@ -199,7 +200,7 @@ def traffic(cfg_id: int, d: Path, copy_dir: Path, commit: str) -> None:
     run = f"python3 bench.py --config {cfg_id} --configs none --steps 2 --warmup 1 --no-cpu-baseline"
     lines = [
         f"# HBM traffic per launch — MoE layer fwd+bwd, {title}", "",
-        f"Measured on the kernels of commit `{commit}` (kernel source hash "
+        f"Measured on a tree that stood on commit `{commit}` (kernel source hash "
         f"`{kernel_source_hash()}`). Commands (run from the repository root on one MI355X; "
         "each counter in its own pass):", "", "```",
         f"rocprofv3 --pmc FETCH_SIZE --output-format csv -d {d}/fetch -o {c} -- {run}",
@@ -311,7 +312,7 @@ def kernel_trace(cfg_id: int, d: Path, commit: str, steps: int, bench_log: Path,
     with open(_find(d / "kt", "kernel_stats.csv")) as fh:
         rows = list(csv.DictReader(fh))
     lines = [f"# Kernel trace — MoE layer fwd+bwd, {title}", "",
-             f"Measured on the kernels of commit `{commit}` (kernel source hash "
+             f"Measured on a tree that stood on commit `{commit}` (kernel source hash "
              f"`{kernel_source_hash()}`). Command (run from the repository root on one MI355X):",
              "", "```", cmd, "```", "",
              f"{steps} layer steps. Per-kernel statistics from the `--stats` summary "
@@ -355,7 +356,7 @@ def main() -> None:
     ap.add_argument("--dir", type=Path, required=True,
                     help="folder holding the kt/, fetch/, write/, mfma/ rocprofv3 outputs")
     ap.add_argument("--copy-dir", type=Path, help="folder with copy_fetch/ and copy_write/")
-    ap.add_argument("--commit", required=True, help="commit whose kernels were profiled")
+    ap.add_argument("--commit", required=True, help="commit the profiled tree stands on")
     ap.add_argument("--steps", type=int, default=30, help="layer steps of the kernel trace run")
     ap.add_argument("--kt-cmd", default="", help="the kernel trace command, for the summary")
     args = ap.parse_args()

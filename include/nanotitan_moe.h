@@ -287,6 +287,14 @@ int nt_router_linear_backward(int dtype, const void* x, const float* W, const fl
                               const float* da, int64_t T, int32_t E, int64_t d, void* dx,
                               float* dW, void* ws, size_t ws_bytes, hipStream_t stream);
 
+/* nt_router_linear_backward with x and dx of types of their own: x f32 and dx
+ * f32, f16 or bf16 (for a caller that keeps the cast tokens the linear read),
+ * or both of one type. */
+int nt_router_linear_backward_mixed(int x_dtype, int dx_dtype, const void* x, const float* W,
+                                    const float* dl, const float* da, int64_t T, int32_t E,
+                                    int64_t d, void* dx, float* dW, void* ws, size_t ws_bytes,
+                                    hipStream_t stream);
+
 /* ------------------------------------------------------------- grouped GEMM */
 
 /* Workspace for nt_grouped_gemm_dw and the paired dW + dX calls with these

@@ -109,6 +109,10 @@ EXPORTS: dict[str, tuple[object, list[object]]] = {
         c_int,
         [c_int, _P, _P, _P, _P, c_int64, c_int32, c_int64, _P, _P, _P, c_size_t, _P],
     ),
+    "nt_router_linear_backward_mixed": (
+        c_int,
+        [c_int, c_int, _P, _P, _P, _P, c_int64, c_int32, c_int64, _P, _P, _P, c_size_t, _P],
+    ),
     "nt_grouped_gemm_workspace_bytes": (c_size_t, [c_int, c_int32, c_int64, c_int64, c_int64]),
     "nt_grouped_gemm_tail_workspace_bytes": (
         c_size_t,

@@ -202,17 +202,21 @@ constexpr int kTok = 64;  // tokens whose gradients a workgroup holds in LDS at 
 // dx[t,:] = dl[t,:] W and partial sums of dW = (dl + da)^T x over this
 // workgroup's tokens. A thread owns VEC columns of W (E x VEC registers) and
 // of dW; cg column threads side by side, the 256 / cg groups of them take
-// every (256 / cg)-th token. x is read once, dx written once.
-template <typename T, int EM, int VEC>
+// every (256 / cg)-th token. x (T) is read once, dx (TD) written once.
+template <typename T, typename TD, int EM, int VEC>
 __global__ void __launch_bounds__(kThreads)
 router_linear_backward_kernel(const typename elem<T>::storage* __restrict__ x,
                               const float* __restrict__ W, const float* __restrict__ dl,
                               const float* __restrict__ da, int64_t T_, int32_t E, int64_t d,
-                              int32_t cg, int32_t groups, typename elem<T>::storage* __restrict__ dx,
+                              int32_t cg, int32_t groups, typename elem<TD>::storage* __restrict__ dx,
                               float* __restrict__ partial) {
   typedef typename elem<T>::storage S;
+  typedef typename elem<TD>::storage SD;
   struct alignas(sizeof(S) * VEC) Pack {
     S v[VEC];
+  };
+  struct alignas(sizeof(SD) * VEC) PackD {
+    SD v[VEC];
   };
   __shared__ float s_gx[kTok][EM], s_gw[kTok][EM];
   const int tid = threadIdx.x;
@@ -266,15 +270,15 @@ router_linear_backward_kernel(const typename elem<T>::storage* __restrict__ x,
           }
         }
         if (dx != nullptr) {
-          Pack r;
+          PackD r;
 #pragma unroll
           for (int v = 0; v < VEC; ++v) {
             float z = 0.f;
 #pragma unroll
             for (int e = 0; e < EM; ++e) z = fmaf(s_gx[t][e], w[e][v], z);
-            r.v[v] = elem<T>::store(z);
+            r.v[v] = elem<TD>::store(z);
           }
-          *reinterpret_cast<Pack*>(dx + (t0 + t) * d + c0) = r;
+          *reinterpret_cast<PackD*>(dx + (t0 + t) * d + c0) = r;
         }
       }
     }
@@ -325,20 +329,22 @@ LinearPlan linear_plan(int64_t T, int64_t d, int vec) {
   return p;
 }
 
-template <typename T>
+template <typename T, typename TD>
 int run_linear_backward(const void* x, const float* W, const float* dl, const float* da, int64_t T_,
                         int32_t E, int64_t d, void* dx, float* dW, float* ws, hipStream_t s) {
   typedef typename elem<T>::storage S;
-  const uintptr_t al = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(dx);
-  const int vec = d % 2 == 0 && al % (2 * sizeof(S)) == 0 ? 2 : 1;
+  typedef typename elem<TD>::storage SD;
+  const bool aligned = reinterpret_cast<uintptr_t>(x) % (2 * sizeof(S)) == 0 &&
+                       reinterpret_cast<uintptr_t>(dx) % (2 * sizeof(SD)) == 0;
+  const int vec = d % 2 == 0 && aligned ? 2 : 1;
   const LinearPlan p = linear_plan(T_, d, vec);
   if (p.cols > 65535) return NT_ERR_TOO_LARGE;
   const dim3 grid((unsigned)p.blocks, (unsigned)p.cols);
   float* part = dW != nullptr ? ws : nullptr;
 #define NT_RLB(EM, VEC)                                                                           \
-  hipLaunchKernelGGL((router_linear_backward_kernel<T, EM, VEC>), grid, dim3(kThreads), 0, s,     \
+  hipLaunchKernelGGL((router_linear_backward_kernel<T, TD, EM, VEC>), grid, dim3(kThreads), 0, s,     \
                      static_cast<const S*>(x), W, dl, da, T_, E, d, p.cg, p.groups,               \
-                     static_cast<S*>(dx), part)
+                     static_cast<SD*>(dx), part)
 #define NT_RLB_V(EM) \
   do {               \
     if (vec == 2) NT_RLB(EM, 2); \
@@ -435,9 +441,10 @@ size_t nt_router_linear_backward_workspace_bytes(int64_t T, int32_t E, int64_t d
   return need;
 }
 
-int nt_router_linear_backward(int dtype, const void* x, const float* W, const float* dl,
-                              const float* da, int64_t T, int32_t E, int64_t d, void* dx, float* dW,
-                              void* ws, size_t ws_bytes, hipStream_t stream) {
+int nt_router_linear_backward_mixed(int x_dtype, int dx_dtype, const void* x, const float* W,
+                                    const float* dl, const float* da, int64_t T, int32_t E,
+                                    int64_t d, void* dx, float* dW, void* ws, size_t ws_bytes,
+                                    hipStream_t stream) {
   if (T < 1 || E < 1 || d < 1) return NT_ERR_INVALID_ARG;
   if (E > kMaxLinearExperts) return NT_ERR_TOO_MANY_EXPERTS;
   if (x == nullptr || W == nullptr) return NT_ERR_INVALID_ARG;
@@ -445,12 +452,31 @@ int nt_router_linear_backward(int dtype, const void* x, const float* W, const fl
       (ws == nullptr || ws_bytes < nt_router_linear_backward_workspace_bytes(T, E, d)))
     return NT_ERR_WORKSPACE;
   float* wp = static_cast<float*>(ws);
-  switch (dtype) {
-    case NT_F32: return run_linear_backward<float>(x, W, dl, da, T, E, d, dx, dW, wp, stream);
-    case NT_F16: return run_linear_backward<f16>(x, W, dl, da, T, E, d, dx, dW, wp, stream);
-    case NT_BF16: return run_linear_backward<bf16>(x, W, dl, da, T, E, d, dx, dW, wp, stream);
+  auto run = [&](auto tx, auto td) {
+    return run_linear_backward<decltype(tx), decltype(td)>(x, W, dl, da, T, E, d, dx, dW, wp,
+                                                           stream);
+  };
+  if (x_dtype == NT_F32) {
+    switch (dx_dtype) {
+      case NT_F32: return run(float(), float());
+      case NT_F16: return run(float(), f16());
+      case NT_BF16: return run(float(), bf16());
+      default: return NT_ERR_DTYPE;
+    }
+  }
+  if (x_dtype != dx_dtype) return NT_ERR_DTYPE;
+  switch (x_dtype) {
+    case NT_F16: return run(f16(), f16());
+    case NT_BF16: return run(bf16(), bf16());
     default: return NT_ERR_DTYPE;
   }
+}
+
+int nt_router_linear_backward(int dtype, const void* x, const float* W, const float* dl,
+                              const float* da, int64_t T, int32_t E, int64_t d, void* dx, float* dW,
+                              void* ws, size_t ws_bytes, hipStream_t stream) {
+  return nt_router_linear_backward_mixed(dtype, dtype, x, W, dl, da, T, E, d, dx, dW, ws, ws_bytes,
+                                         stream);
 }
 
 }  // extern "C"

@@ -21,18 +21,19 @@ namespace {
 
 using torch::Tensor;
 
-int dtype_code(const Tensor& t) {
-  switch (t.scalar_type()) {
+int dtype_code(at::ScalarType t) {
+  switch (t) {
     case at::kFloat: return NT_F32;
     case at::kDouble: return NT_F64;
     case at::kHalf: return NT_F16;
     case at::kBFloat16: return NT_BF16;
     default:
-      TORCH_CHECK(false, "unsupported dtype ", t.scalar_type(),
+      TORCH_CHECK(false, "unsupported dtype ", t,
                   " (expected float32, float64, float16 or bfloat16)");
   }
   return -1;
 }
+int dtype_code(const Tensor& t) { return dtype_code(t.scalar_type()); }
 
 at::ScalarType scalar_of(int code) {
   switch (code) {
@@ -833,11 +834,12 @@ Tensor router_stats_backward(Tensor logits, Tensor frac, c10::optional<Tensor> d
   return out;
 }
 
-// router_linear_backward(x, W, dl, da, need_dx, need_dW) -> (dx, dW): dx = dl W,
-// dW = (dl + da)^T x; a missing gradient is zero, an output not needed undefined.
+// router_linear_backward(x, W, dl, da, need_dx, need_dW, dx_dtype=x's) -> (dx, dW):
+// dx = dl W, dW = (dl + da)^T x; a missing gradient is zero, an output not needed
+// undefined. dx_dtype may differ from x's where x is float32.
 std::tuple<c10::optional<Tensor>, c10::optional<Tensor>> router_linear_backward(
     Tensor x, Tensor W, c10::optional<Tensor> dl, c10::optional<Tensor> da, bool need_dx,
-    bool need_dW) {
+    bool need_dW, c10::optional<at::ScalarType> dx_dtype) {
   check_device(x, "x");
   check_f32(W, "weight");
   TORCH_CHECK(x.is_contiguous() && W.is_contiguous(), "inputs must be contiguous");
@@ -855,12 +857,13 @@ std::tuple<c10::optional<Tensor>, c10::optional<Tensor>> router_linear_backward(
   }
   c10::hip::HIPGuard guard(x.get_device());
   c10::optional<Tensor> dx, dW;
-  if (need_dx) dx = at::empty_like(x);
+  const at::ScalarType dxt = dx_dtype.value_or(x.scalar_type());
+  if (need_dx) dx = at::empty_like(x, x.options().dtype(dxt));
   if (need_dW) dW = at::empty_like(W);
   Tensor ws = workspace(
       x, need_dW ? nt_router_linear_backward_workspace_bytes(T, (int32_t)E, d) : 0);
-  check_status(nt_router_linear_backward(
-                   dtype_code(x), x.data_ptr(), W.data_ptr<float>(),
+  check_status(nt_router_linear_backward_mixed(
+                   dtype_code(x), dtype_code(dxt), x.data_ptr(), W.data_ptr<float>(),
                    dl ? dl->data_ptr<float>() : nullptr, da ? da->data_ptr<float>() : nullptr, T,
                    (int32_t)E, d, need_dx ? dx->data_ptr() : nullptr,
                    need_dW ? dW->data_ptr<float>() : nullptr, ws.data_ptr(), ws.numel(),
@@ -1205,7 +1208,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("router_stats_backward", &router_stats_backward,
         "Gradient of router_stats' aux and mean to the logits");
   m.def("router_linear_backward", &router_linear_backward,
-        "Backward of the router's linear layer for both of its gradients -> (dx, dW)");
+        "Backward of the router's linear layer for both of its gradients -> (dx, dW)",
+        pybind11::arg("x"), pybind11::arg("weight"), pybind11::arg("dl"), pybind11::arg("da"),
+        pybind11::arg("need_dx"), pybind11::arg("need_dW"), pybind11::arg("dx_dtype") = pybind11::none());
   m.def("stream_fill", &stream_fill, "16-byte streaming device fill (write bandwidth reference)",
         pybind11::arg("dst"), pybind11::arg("value") = 0);
   m.def("stream_read", &stream_read, "16-byte streaming device read (read bandwidth reference)",

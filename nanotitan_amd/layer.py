@@ -82,7 +82,7 @@ class MoELayerStats:
     def from_logits(cls, tokens_per_expert, logits, cfg, router=None):
         """The same statistics from the float32 router logits, in one kernel.
 
-        ``router``: (tokens, weight) where the gradient goes to the weight of
+        ``router``: (float32 tokens, weight) where the gradient goes to the weight of
         the linear that gives these logits; else it goes to ``logits``.
         """
         stats = cls.__new__(cls)
@@ -212,7 +212,8 @@ class HIPMoEBackend:
             grad = torch.is_grad_enabled()
             one_pass = plain and (not grad or self.router.weight.shape[0] <= 32)
             if one_pass and grad:
-                logits = router_gate_fn(flat, self.router.weight)
+                flat32 = flat.to(router_dtype)
+                logits = router_gate_fn(flat, flat32, self.router.weight)
             else:
                 logits = self.router(flat.to(router_dtype))
         if one_pass:
@@ -225,7 +226,7 @@ class HIPMoEBackend:
         if plain:
             stats = MoELayerStats.from_logits(
                 counts.detach(), aux_logits, self.cfg,
-                router=(flat, self.router.weight) if one_pass and grad else None)
+                router=(flat32, self.router.weight) if one_pass and grad else None)
         else:
             stats = MoELayerStats(tokens_per_expert=counts.detach(),
                                   probs_per_expert=aux_logits.softmax(dim=-1), cfg=self.cfg)

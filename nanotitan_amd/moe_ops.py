@@ -408,29 +408,34 @@ class RouteDispatchFN(torch.autograd.Function):
 
 
 class RouterGateFN(torch.autograd.Function):
-    """The router's logits x @ weight.T (float32) for the gate path.
+    """The router's logits x32 @ weight.T (float32) for the gate path.
 
-    x [T,d], weight [E,d] float32, E <= 32. One kernel gives dx = dl W and
-    dW = dl^T x (reference src/model/cuda_backend.py:27-30).
+    x [T,d], x32 the same in float32, weight [E,d] float32, E <= 32. One
+    kernel gives dx = dl W in x's dtype and dW = dl^T x (reference
+    src/model/cuda_backend.py:27-30). What is saved is x32, as the linear on
+    the cast tokens saves it: a 16-bit x may be written to after the forward
+    (an in-place residual).
     """
 
     @staticmethod
-    def forward(ctx, x, weight):
-        ctx.save_for_backward(x, weight)
+    def forward(ctx, x, x32, weight):
+        ctx.save_for_backward(x32, weight)
+        ctx.x_dtype = x.dtype
         ctx.set_materialize_grads(False)
-        return torch.nn.functional.linear(x.to(weight.dtype), weight)
+        return torch.nn.functional.linear(x32, weight)
 
     @staticmethod
     def backward(ctx, dl):
-        x, weight = ctx.saved_tensors
-        need_dx, need_dW = ctx.needs_input_grad
+        x32, weight = ctx.saved_tensors
+        need_dx, need_dx32, need_dW = ctx.needs_input_grad
         if dl is None:
-            return None, None
-        if torch.is_grad_enabled():  # differentiated again: composed of torch ops
-            return ((dl @ weight).to(x.dtype) if need_dx else None,
-                    dl.t() @ x.to(weight.dtype) if need_dW else None)
-        return get_hip_extension().router_linear_backward(
-            x.contiguous(), weight.contiguous(), dl.contiguous(), None, need_dx, need_dW)
+            return None, None, None
+        if torch.is_grad_enabled():  # differentiated again: torch ops, dx through the cast
+            return (None, dl @ weight if need_dx32 else None, dl.t() @ x32 if need_dW else None)
+        dx, dW = get_hip_extension().router_linear_backward(
+            x32.contiguous(), weight.contiguous(), dl.contiguous(), None, need_dx, need_dW,
+            ctx.x_dtype)
+        return dx, None, dW
 
 
 class RouterStatsFN(torch.autograd.Function):
@@ -483,15 +488,15 @@ class RouterAuxFN(torch.autograd.Function):
     the router's weight. Both passes compute the same logits, so the first
     pass's are taken; the graph is the second pass's own (one of the two can
     be differentiated and freed before the other). logits [T,E] float32 =
-    x @ weight.T, x [T,d] and logits without gradients, E <= 32.
+    x32 @ weight.T, x32 [T,d] float32 and logits without gradients, E <= 32.
     """
 
     @staticmethod
-    def forward(ctx, logits, x, weight, counts, coef):
+    def forward(ctx, logits, x32, weight, counts, coef):
         logits = logits.contiguous()
         total, frac, mean, aux = get_hip_extension().router_stats(logits, counts.contiguous(),
                                                                   coef)
-        ctx.save_for_backward(logits, frac, x, weight)
+        ctx.save_for_backward(logits, frac, x32, weight)
         ctx.coef = coef
         ctx.mark_non_differentiable(total, frac)
         ctx.set_materialize_grads(False)
@@ -499,28 +504,27 @@ class RouterAuxFN(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, _dtotal, _dfrac, dmean, daux):
-        logits, frac, x, weight = ctx.saved_tensors
+        logits, frac, x32, weight = ctx.saved_tensors
         if dmean is None and daux is None:
             return None, None, None, None, None
         if torch.is_grad_enabled():  # differentiated again: composed of torch ops
-            x = x.to(weight.dtype)
-            da = _stats_dlogits(x @ weight.t(), frac, daux, dmean, ctx.coef)
-            return None, None, da.t() @ x, None, None
+            da = _stats_dlogits(x32 @ weight.t(), frac, daux, dmean, ctx.coef)
+            return None, None, da.t() @ x32, None, None
         ext = get_hip_extension()
         da = ext.router_stats_backward(logits, frac, None if daux is None else daux.contiguous(),
                                        None if dmean is None else dmean.contiguous(), ctx.coef)
-        _, dW = ext.router_linear_backward(x.contiguous(), weight.contiguous(), None, da, False,
-                                           True)
+        _, dW = ext.router_linear_backward(x32.contiguous(), weight.contiguous(), None, da,
+                                           False, True)
         return None, None, dW, None, None
 
 
-def router_gate_fn(x, weight):
-    return RouterGateFN.apply(x, weight)
+def router_gate_fn(x, x32, weight):
+    return RouterGateFN.apply(x, x32, weight)
 
 
-def router_aux_fn(logits, x, weight, counts, coef):
-    """Statistics of RouterStatsFN; logits and x are used without their gradients."""
-    return RouterAuxFN.apply(logits.detach(), x.detach(), weight, counts, coef)
+def router_aux_fn(logits, x32, weight, counts, coef):
+    """Statistics of RouterStatsFN; logits and x32 are used without their gradients."""
+    return RouterAuxFN.apply(logits.detach(), x32.detach(), weight, counts, coef)
 
 
 def router_stats_fn(logits, counts, coef):

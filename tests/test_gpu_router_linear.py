@@ -148,3 +148,47 @@ def test_loss_and_output_have_graphs_of_their_own(ext, E):
     y, st = moe(x)
     assert y.requires_grad and not st.aux_loss.requires_grad
     assert not st.probs_per_expert.requires_grad
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_tokens_may_be_overwritten_after_the_forward(ext, dtype):
+    """An in-place residual: the layer keeps the cast tokens, not x."""
+    moe, x = _moe(8, dtype)
+    params = list(moe.parameters())
+
+    def step(in_place):
+        leaf = x.clone().requires_grad_()
+        h = leaf * 1
+        y, st = moe(h)
+        if in_place:
+            h += y
+        else:
+            h = h + y
+        return torch.autograd.grad(h.float().square().sum() + st.aux_loss, [leaf, *params])
+
+    for a, b in zip(step(True), step(False)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,E,d,shift", [(5, 3, 7, 0), (65, 16, 130, 0), (130, 17, 64, 1)])
+def test_router_linear_backward_from_float32(ext, dtype, T, E, d, shift):
+    """x in float32, dx in the tokens' type: the bits of x in that type. Off
+    8-byte alignment (shift) one column a thread divides the tokens otherwise,
+    so dW is summed in another order: the bound of a sum of T products."""
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, d, generator=g).to(dtype)
+    W, dl = torch.randn(E, d, generator=g).cuda(), torch.randn(T, E, generator=g).cuda()
+    buf = torch.empty(T * d + shift, device="cuda")
+    buf[shift:] = x.float().reshape(-1).cuda()
+    got = ext.router_linear_backward(buf[shift:].view(T, d), W, dl, None, True, True, dtype)
+    ref = ext.router_linear_backward(x.cuda(), W, dl, None, True, True)
+    assert got[0].dtype == dtype
+    assert torch.equal(got[0], ref[0])
+    if shift == 0:
+        assert torch.equal(got[1], ref[1])
+    dld, xd = dl.cpu().double(), x.double()
+    bound = (T + 8) * 2.0**-24 * (dld.abs().t() @ xd.abs())
+    assert bool(((got[1].cpu().double() - dld.t() @ xd).abs() <= bound).all())
+    with pytest.raises(RuntimeError):  # only float32 tokens may differ from their gradient
+        ext.router_linear_backward(x.cuda(), W, dl, None, True, True, torch.float32)
