@@ -23,12 +23,17 @@ namespace {
 // fp32 runs on the bf16 MFMA: each value is the sum of three bf16 terms
 // (x = h + m + l, each the round-to-nearest of what is left: 24 bits), and
 // a product is the six term products down to 2^-18 (h l, m m, l h, then
-// h m, m h, h h) in fp32 accumulators; the dropped ones are below 2^-26 of
-// the product. Six products on a matrix core that runs bf16 at 16 times
-// the fp32 rate. A tile with a non-finite result is reduced again with
-// v_mfma_f32_16x16x4 on the unsplit values: an infinite operand has no
-// finite remainder to split, so only that keeps inf and NaN as fp32
-// arithmetic gives them.
+// h m, m h, h h) in fp32 accumulators; the dropped ones (m l, l m: each up
+// to 2^-25; l l) are below 2^-24 of the product, one fp32 rounding. Six
+// products on a matrix core that runs bf16 at 16 times the fp32 rate. Two
+// kinds of tile are reduced again with v_mfma_f32_16x16x4 on the unsplit
+// values: one with a non-finite result (an infinite operand has no finite
+// remainder to split, so only that keeps inf and NaN as fp32 arithmetic
+// gives them), and one with an operand that the three terms do not hold: below
+// 2^-110 its last bits lie under bf16's smallest subnormal, 2^-133 (the bf16
+// MFMA keeps subnormal operands). Measured on MI355X, 132-term sums, largest
+// error over sum |a||b|: 9.5e-8 down to 2^-110; split below it 2.2e-6 at 2^-118
+// and 5.7e-4 at 2^-126, unsplit 1.3e-7 throughout.
 //
 // 128x128 outputs, 4 waves of 64x64, one LDS stage of 32 KiB (16-bit, 64
 // deep) or 48 KiB (fp32, 32 deep): two (fp32) or three (16-bit) workgroups
@@ -184,7 +189,9 @@ struct StagedTile {
     }
   }
   // Write the chunks to LDS: as they are (16-bit), or as three bf16 planes.
-  __device__ void store(char* smem, const uint4 (&reg)[kPer][kWords]) const {
+  // The third term is exact if what the first two leave is a bf16 value, the
+  // upper half of an fp32 one: `lost` collects the bits of the lower halves.
+  __device__ void store(char* smem, const uint4 (&reg)[kPer][kWords], uint32_t& lost) const {
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
       char* p = smem + lds + u * kRowStep * kRowBytes;
@@ -199,6 +206,7 @@ struct StagedTile {
           float a = x[2 * i], b = x[2 * i + 1];
 #pragma unroll
           for (int pl = 0; pl < 3; ++pl) {
+            if (pl == 2) lost |= __float_as_uint(a) | __float_as_uint(b);
             t[pl][i] = pack2<bf16>(a, b);
             a -= __uint_as_float(t[pl][i] << 16);
             b -= __uint_as_float(t[pl][i] & 0xffff0000u);
@@ -413,6 +421,7 @@ gg_staged_kernel(GemmArgs g) {
   fb[1].init(kHalves ? 64 + wn * 32 : wn * 64 + 32, lane);
   typedef typename mfma_op<M>::vec vec;
 
+  uint32_t lost = 0;
   if (kb < ke) fetch(kb);
   for (int64_t kt = kb; kt < ke; ++kt) {
     __syncthreads();  // the stage's readers are done
@@ -421,8 +430,8 @@ gg_staged_kernel(GemmArgs g) {
       ta.mask(left, ra);
       tb.mask(left, rb);
     }
-    ta.store(sa, ra);
-    tb.store(sb, rb);
+    ta.store(sa, ra, lost);
+    tb.store(sb, rb, lost);
     __syncthreads();
     if (kt + 1 < ke) fetch(kt + 1);
 #pragma unroll
@@ -465,7 +474,7 @@ gg_staged_kernel(GemmArgs g) {
     return kHalves ? wn * 32 + acc_col(q, lane) : wn * 64 + j * 32 + acc_col(q, lane);
   };
   if constexpr (NP == 3) {
-    bool bad = false;
+    bool bad = (lost & 0xffffu) != 0;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll

@@ -3,7 +3,7 @@ rows are not whole aligned 16-byte chunks) against float64.
 
 Bound, per element: a reduction of length R over products rounded to fp32
 errs by at most (R + 8) 2^-24 sum |a||b| (any summation order; the 8 covers
-fp32's split operands, whose dropped terms are below 2^-25 of a product), and
+fp32's split operands, whose dropped terms are below 2^-24 of a product), and
 the result is rounded once more to its own type of p significant bits, by at
 most 2^-p of its value (p = 8 bf16, 11 fp16, 24 fp32), or 2^-25 at fp16's
 subnormals."""
@@ -122,3 +122,45 @@ def test_staged_f32_non_finite(ext, mode):
     ok = torch.isfinite(ref)
     assert torch.equal(out[torch.isinf(ref)], ref[torch.isinf(ref)])
     torch.testing.assert_close(out[ok], ref[ok], rtol=1e-4, atol=1e-3)
+
+
+@pytest.mark.parametrize("mode", ["fwd", "dX", "dW"])
+@pytest.mark.parametrize("R", [1, 132])
+@pytest.mark.parametrize("ex,ew,rows", [
+    (-110, 0, None), (-111, 0, None), (-114, 0, None), (-126, 0, None), (0, -114, None),
+    (0, -126, None), (-126, 60, None), (-60, -60, None), (-118, 0, 3)])
+def test_staged_f32_small_operands(ext, mode, R, ex, ew, rows):
+    """Operands whose last bits no third bf16 term holds (below 2^-110) keep
+    24 bits: the same relative bound at every magnitude, without an absolute
+    term (products of values in [2^e, 2^(e+1)) stay normal here). rows: only
+    that row of the left operand is small, between ordinary ones. A sum of one
+    product (R = 1) shows a loss from 2^-114 on, long sums from 2^-126."""
+    g = torch.Generator().manual_seed(6)
+    A, K, N = 200, 132, 140
+    A, K, N = {"fwd": (A, R, N), "dX": (A, K, R), "dW": (R, K, N)}[mode]
+    offsets = torch.tensor([0, A], dtype=torch.int32, device="cuda")
+
+    def values(*shape):
+        return torch.randn(shape, generator=g).sign() * (1 + torch.rand(shape, generator=g))
+
+    a, b = {"fwd": ((A, K), (K, N)), "dX": ((A, N), (K, N)), "dW": ((A, K), (A, N))}[mode]
+    a, b = values(*a), values(*b)
+    b = torch.ldexp(b, torch.tensor(ew))
+    if rows is None:
+        a = torch.ldexp(a, torch.tensor(ex))
+    elif mode == "dW":
+        a[:, rows] = torch.ldexp(a[:, rows], torch.tensor(ex))
+    else:
+        a[rows] = torch.ldexp(a[rows], torch.tensor(ex))
+    ad, bd = a.double(), b.double()
+    if mode == "fwd":
+        out = ext.grouped_gemm_kernel(a.cuda(), offsets, b.cuda()[None])
+        ref, mag = ad @ bd, ad.abs() @ bd.abs()
+    elif mode == "dX":
+        out = ext.bwd_grouped_gemm_dX_kernel(b.cuda()[None], offsets, a.cuda())
+        ref, mag = ad @ bd.t(), ad.abs() @ bd.abs().t()
+    else:
+        out = ext.bwd_grouped_gemm_dW_kernel(a.cuda(), offsets, b.cuda())[0]
+        ref, mag = ad.t() @ bd, ad.abs().t() @ bd.abs()
+    err = (out.cpu().double() - ref).abs()
+    assert bool((err <= (R + 8) * 2.0**-24 * mag).all()), float((err / mag).max())

@@ -93,3 +93,28 @@ def test_tail_pieces_under_graph_replay(ext, dtype, K, N):
         eager = ext.grouped_gemm_kernel(Xg, og, Wg)
         torch.cuda.synchronize()
         assert torch.equal(out, eager), seed
+
+
+@pytest.mark.parametrize("K,N", [(512, 130), (1001, 64)])
+def test_tail_pieces_f32_special_values(ext, K, N):
+    """The fp32 repair (non-finite results, operands below 2^-110) runs per piece:
+    values of one k index each, so that other pieces of their tile are ordinary."""
+    offs, X, W, seg = _case(torch.float32, K, N, seed=3)
+    E, A = W.shape[0], X.shape[0]
+    assert capi.load().nt_grouped_gemm_tail_workspace_bytes(capi.dtype_code(X.dtype), 0, E, A, K,
+                                                            N) > 0
+    W.clamp_(-0.9, 0.9)
+    X[3, 5] = float("inf")
+    X[131, K - 1] = float("nan")
+    X[250, 7] = 3.4e38  # finite in fp32, rounds to infinity in bf16
+    X[400] = torch.ldexp(X[400], torch.tensor(-120))
+    out = ext.grouped_gemm_kernel(X.cuda(), offs.cuda(), W.cuda())
+    out = out.cpu()
+    ref = torch.cat([X[s].double() @ W[e].double() for e, s in seg])
+    mag = torch.cat([X[s].double().abs() @ W[e].double().abs() for e, s in seg])
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    inf = torch.isinf(ref)
+    assert torch.equal(torch.isinf(out), inf) and torch.equal(out[inf], ref[inf].float())
+    ok = torch.isfinite(ref)
+    err = (out.double() - ref).abs()
+    assert bool((err[ok] <= (K + 8) * 2.0**-24 * mag[ok] + 2.0**-24 * ref[ok].abs()).all())
