@@ -1530,6 +1530,19 @@ constexpr int64_t kFewRows = 32, kFewRowsSwiGLU = 48;
 // (the last layer's weights stay in the cache: only its SwiGLU gains).
 constexpr int64_t kMidRows = 112;
 constexpr int64_t kStreamedBytes = int64_t(256) << 20;
+// The tile rules of forward and dX launches, shared with the tail split's
+// (tail_bytes: only 128x128 tiles are cut). 64-row tiles for few rows per
+// expert, 128x256 ones up to kMidRows where the weights are streamed, 256x256
+// ones where they make 1.5 rounds, else 128x128.
+bool rows_per_expert_at_most(int64_t A, int32_t E, int64_t rows) {
+  return A <= rows * std::min<int64_t>(E, A);  // of the experts that can have rows
+}
+bool mid_rows_streamed(int64_t A, int32_t E, int64_t K, int64_t N) {
+  return rows_per_expert_at_most(A, E, kMidRows) &&
+         std::min<int64_t>(E, A) * K * N * 2 > kStreamedBytes;
+}
+bool fills_256_tiles(int64_t tiles256, int64_t cus) { return tiles256 * 2 >= cus * 3; }
+
 template <int MODE, int EPI>
 int launch_mfma_auto(int dtype, GemmArgs g, int64_t out_cols, hipStream_t s) {
   const int64_t chunks = g.chunk > 0 ? g.E + g.A / g.chunk : g.E;
@@ -1538,29 +1551,28 @@ int launch_mfma_auto(int dtype, GemmArgs g, int64_t out_cols, hipStream_t s) {
                                : ceil_div(g.A, 256) * ceil_div(out_cols, 256);
   // Few rows per expert (decode): the weights' bytes bound the launch, so the
   // tiles are 64 rows high and the LDS holds three stages of them.
-  const int64_t experts = std::min<int64_t>(g.E, g.A);  // that can have rows
-  const bool few_rows =
-      MODE != kDw && g.A <= (EPI == kEpiSwiGLU ? kFewRowsSwiGLU : kFewRows) * experts;
-  const bool mid_rows = MODE != kDw && g.A <= kMidRows * experts;
+  const bool few_rows = MODE != kDw && rows_per_expert_at_most(
+                                           g.A, g.E, EPI == kEpiSwiGLU ? kFewRowsSwiGLU : kFewRows);
   // SwiGLU forward: 256 rows x (128 gate | 128 value) columns, waves 4 x 2,
   // so that each wave holds the gate and value tiles of the same outputs.
   if constexpr (EPI == kEpiSwiGLU) {
     (void)tiles256;
     if (few_rows) return launch_mfma<MODE, EPI, 64, 256, 2, 2, 64, 3>(dtype, g, out_cols, s);
-    if (mid_rows) return launch_mfma<MODE, EPI, 128, 256, 4, 2, 64, 3>(dtype, g, out_cols, s);
+    if (rows_per_expert_at_most(g.A, g.E, kMidRows))
+      return launch_mfma<MODE, EPI, 128, 256, 4, 2, 64, 3>(dtype, g, out_cols, s);
     return launch_mfma<MODE, EPI, 256, 256, 4, 2, 64, 2>(dtype, g, out_cols, s);
   } else {
     if constexpr (MODE != kDw && (EPI == kEpiPlain || EPI == kEpiGelu)) {
       if (few_rows) {
-        if (experts * ceil_div(out_cols, 256) * 2 > (int64_t)device_cus(s) * 3)
+        if (std::min<int64_t>(g.E, g.A) * ceil_div(out_cols, 256) * 2 > (int64_t)device_cus(s) * 3)
           return launch_mfma<MODE, EPI, 64, 256, 2, 2, 64, 3>(dtype, g, out_cols, s);
         return launch_mfma<MODE, EPI, 64, 128, 2, 2, 64, 3>(dtype, g, out_cols, s);
       }
-      if (mid_rows && experts * g.K * g.N * 2 > kStreamedBytes)
+      if (mid_rows_streamed(g.A, g.E, g.K, g.N))
         return launch_mfma<MODE, EPI, 128, 256, 2, 4, 64, 3>(dtype, g, out_cols, s);
     }
     constexpr bool kTail = MODE == kDx || (MODE == kFwd && EPI == kEpiPlain);
-    if (tiles256 * 2 >= (int64_t)device_cus(s) * 3) {
+    if (fills_256_tiles(tiles256, device_cus(s))) {
       if constexpr (MODE != kDw && (EPI == kEpiPlain || EPI == kEpiDualK)) {
         const int64_t red = MODE == kFwd ? g.K : (EPI == kEpiDualK ? 2 * g.N : g.N);
         if (red >= kSplitMinRed)
@@ -2002,7 +2014,9 @@ bool pair_shape(int32_t E, int64_t K, int64_t N, int64_t cus) {
 // many k-steps each) and which are a few rounds of tiles at most. Not the
 // shapes that run paired with their dW: a separate dX is bit-equal to that.
 // A dX is cut the same way with and without a fused activation, whose values
-// stay those of the activation applied to the separate dX.
+// stay those of the activation applied to the separate dX: the rule is that
+// of the plain dX, also at few rows per expert, where a fused one runs on
+// 128x128 tiles like these but the plain one on 64-row tiles, never cut.
 // The GEMMs of wide outputs stay whole, so the SwiGLU forward's gate and
 // value are the separate GEMMs' bits there. Measured on MI355X, whole tiles
 // to cut: bf16, two-part dX over 2 x 2048 to 512 for 16 experts: 4,096 rows
@@ -2013,7 +2027,8 @@ bool pair_shape(int32_t E, int64_t K, int64_t N, int64_t cus) {
 constexpr int32_t kTailSlots = 512;
 constexpr size_t kTailCtrBytes = kTailSlots * 8;
 constexpr size_t kTailBytes = kTailCtrBytes + (size_t)kTailSlots * 128 * 128 * 4;
-size_t tail_bytes(int op, int dtype, int32_t E, int64_t A, int64_t K, int64_t N) {
+size_t tail_bytes(int op, int dtype, int32_t E, int64_t A, int64_t K, int64_t N,
+                  int64_t device_cus) {
   if (dtype_bytes(dtype) == 0 || dtype == NT_F64 || E < 1 || A < 1 || K < 1 || N < 1) return 0;
   const int64_t red = op == NT_GEMM_FWD ? K : N, out = op == NT_GEMM_FWD ? N : K;
   if (red <= out || red < 512) return 0;
@@ -2023,13 +2038,24 @@ size_t tail_bytes(int op, int dtype, int32_t E, int64_t A, int64_t K, int64_t N)
   if (dtype != NT_F32 && K % 8 == 0 && N % 8 == 0 && red * (op == NT_GEMM_DX2 ? 2 : 1) <= 2048)
     return 0;
   if (op != NT_GEMM_FWD && dtype != NT_F32 && K % 8 == 0 && N % 8 == 0 &&
-      pair_shape(E, K, N, kDwSplitCus))
+      pair_shape(E, K, N, device_cus))
     return 0;
+  if (dtype != NT_F32 && K % 8 == 0 && N % 8 == 0 && (op != NT_GEMM_DX2 || N % 64 == 0)) {
+    // launch_mfma_auto on these sizes: cut only where it takes 128x128 tiles
+    if (op != NT_GEMM_DX2 &&
+        (rows_per_expert_at_most(A, E, kFewRows) || mid_rows_streamed(A, E, K, N)))
+      return 0;
+    if (fills_256_tiles(ceil_div(A, 256) * ceil_div(out, 256), device_cus)) return 0;
+  } else {
+    GemmArgs g{};
+    g.E = E, g.A = A, g.K = K, g.N = N;
+    if (!staged_ok(op == NT_GEMM_FWD ? kFwd : kDx, dtype, g)) return 0;
+  }
   const int64_t tiles = (ceil_div(A, 128) + std::min<int64_t>(E, A)) * ceil_div(out, 128);
   return tiles <= 4 * 2 * kDwSplitCus ? kTailBytes : 0;
 }
 int attach_tail(GemmArgs& g, int op, int dtype, void* ws, size_t ws_bytes, hipStream_t stream) {
-  const size_t need = tail_bytes(op, dtype, g.E, g.A, g.K, g.N);
+  const size_t need = tail_bytes(op, dtype, g.E, g.A, g.K, g.N, device_cus(stream));
   if (need == 0 || ws == nullptr || ws_bytes < need || reinterpret_cast<uintptr_t>(ws) % 16 != 0)
     return NT_OK;
   g.tail_slots = kTailSlots;
@@ -2151,7 +2177,7 @@ size_t nt_grouped_gemm_workspace_bytes(int dtype, int32_t E, int64_t A, int64_t 
 size_t nt_grouped_gemm_tail_workspace_bytes(int dtype, int op, int32_t E, int64_t A, int64_t K,
                                             int64_t N) {
   if (op != NT_GEMM_FWD && op != NT_GEMM_DX && op != NT_GEMM_DX2) return 0;
-  return tail_bytes(op, dtype, E, A, K, N);
+  return tail_bytes(op, dtype, E, A, K, N, kDwSplitCus);
 }
 
 int nt_grouped_gemm(int dtype, const void* X, const int32_t* offsets, const void* W, int32_t E,

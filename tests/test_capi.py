@@ -55,6 +55,31 @@ def test_dispatch_block_tokens():
     assert bt(100, 2, 8, 99) == 0
 
 
+@pytest.mark.parametrize("dtype,op,E,A,K,N,cut", [
+    # op 0: forward K -> N; 1, 2: dX of one / two parts, N -> K
+    ("bf16", 0, 16, 16 * 33, 4096, 512, True),     # 128x128 tiles
+    ("bf16", 0, 16, 16 * 32, 4096, 512, False),    # 64-row tiles
+    ("bf16", 2, 16, 16 * 32, 512, 4096, True),     # the two-part dX has none
+    ("bf16", 0, 32, 32 * 112, 8960, 512, False),   # 128x256: weights past 256 MiB
+    ("bf16", 0, 32, 32 * 113, 8960, 512, True),
+    ("bf16", 1, 32, 32 * 112, 512, 8192, True),    # exactly 256 MiB
+    ("bf16", 1, 17, 49152, 512, 2112, False),      # 256x256: 1.5 rounds
+    ("bf16", 1, 17, 48896, 512, 2112, True),
+    ("bf16", 2, 17, 49152, 512, 2120, True),       # register-staged: 128x128 at any size
+    ("bf16", 1, 8, 8192, 512, 2112, False),        # paired with its dW
+    ("bf16", 0, 16, 16 * 4, 4097, 512, True),      # register-staged
+    ("fp32", 0, 16, 16 * 4, 4096, 512, True),
+    ("fp32", 0, 16, 64, 2**21 + 8, 8, False),      # past its row pitch
+    ("fp64", 0, 16, 16 * 64, 4096, 512, False)])
+def test_tail_workspace_only_where_tiles_may_be_cut(dtype, op, E, A, K, N, cut):
+    import torch
+
+    code = capi.dtype_code({"bf16": torch.bfloat16, "fp32": torch.float32,
+                            "fp64": torch.float64}[dtype])
+    size = capi.load().nt_grouped_gemm_tail_workspace_bytes(code, op, E, A, K, N)
+    assert size == (2**25 + 2**12 if cut else 0)
+
+
 def test_workspace_sizes_are_sane():
     lib = capi.load()
     assert lib.nt_dispatch_workspace_bytes(30720, 2, 8, 512, capi.NT_BF16) > 0

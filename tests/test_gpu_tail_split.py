@@ -118,3 +118,29 @@ def test_tail_pieces_f32_special_values(ext, K, N):
     ok = torch.isfinite(ref)
     err = (out.double() - ref).abs()
     assert bool((err[ok] <= (K + 8) * 2.0**-24 * mag[ok] + 2.0**-24 * ref[ok].abs()).all())
+
+
+# (E, rows per expert, K = dX columns, N = reduction): the plain dX runs on
+# 64-row tiles, on 128x256 ones (weights past 256 MiB), on 256x256 ones
+WHOLE = [(32, 16, 768, 4096), (32, 64, 512, 8960), (17, 2892, 512, 2112)]
+
+
+@pytest.mark.parametrize("E,rows,K,N", WHOLE)
+def test_fused_dx_equals_dx_where_dx_is_not_cut(ext, E, rows, K, N):
+    """The fused dX runs on other tiles there: it is not cut either."""
+    g = torch.Generator(device="cuda").manual_seed(E + K)
+    A = E * rows
+
+    def randn(*shape):
+        return torch.randn(shape, generator=g, device="cuda").to(torch.bfloat16)
+
+    offs = torch.arange(0, A + 1, rows, dtype=torch.int32, device="cuda")
+    W, D, H, V = randn(E, K, N), randn(A, N), randn(A, K), randn(A, K)
+    G = torch.full_like(H, 64)  # silu(64) is 64: dvalue is 64 dX
+    assert capi.load().nt_grouped_gemm_tail_workspace_bytes(capi.dtype_code(W.dtype), 1, E, A, K,
+                                                            N) == 0
+    dX = ext.bwd_grouped_gemm_dX_kernel(W, offs, D)
+    dH = ext.bwd_grouped_gemm_dX_gelu(W, offs, D, H)
+    assert torch.equal(dH, (dX.float() * H.float()).to(W.dtype))
+    assert torch.equal(ext.bwd_grouped_gemm_dX_swiglu(W, offs, D, G, V)[1], 64 * dX)
+    assert torch.equal(ext.bwd_grouped_gemm_dW_dX_gelu(H, W, offs, D, H)[1], dH)
