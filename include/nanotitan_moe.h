@@ -313,14 +313,18 @@ int nt_router_linear_backward_mixed(int x_dtype, int dx_dtype, const void* x, co
 size_t nt_grouped_gemm_workspace_bytes(int dtype, int32_t E, int64_t A, int64_t K, int64_t N);
 
 /* Workspace with which nt_grouped_gemm, nt_grouped_gemm_dx (_gelu, _swiglu)
- * and nt_grouped_gemm_dx2 (and the dX of the dW + dX calls, where larger than
- * nt_grouped_gemm_workspace_bytes) may cut the tiles of a nearly empty last
- * round along the reduction, one piece per idle workgroup, and sum the
- * pieces in order: 0 where these sizes are never cut, else 32 MiB and 4 KiB.
- * Smaller or NULL: no tile is cut. The result is the same to float32 rounding
- * of the sums, and the same bits on every call with such a workspace. Contents
- * and sharing as for nt_grouped_gemm_workspace_bytes. op: the forward, a
- * one-part dX (with any epilogue), or the two-part dX. */
+ * and nt_grouped_gemm_dx2 may cut the tiles of a nearly empty last round along
+ * the reduction, one piece per idle workgroup, and sum the pieces in order: 0
+ * where these sizes are never cut, else 32 MiB and 4 KiB. Smaller or NULL: no
+ * tile is cut. A dW + dX call cuts its dX with this much behind its dW
+ * workspace, that is with nt_grouped_gemm_workspace_bytes rounded up to 256,
+ * plus these bytes. The result is the same to float32 rounding of the sums,
+ * and the same bits on every call with such a workspace; which rows lie in a
+ * cut tile depends on all offsets and on the device's CU count, so a row's
+ * last bits may differ in another batch, where whole tiles give every row the
+ * same bits in any batch. Contents and sharing as for
+ * nt_grouped_gemm_workspace_bytes. op: the forward, a one-part dX (with any
+ * epilogue), or the two-part dX. */
 enum { NT_GEMM_FWD = 0, NT_GEMM_DX = 1, NT_GEMM_DX2 = 2 };
 size_t nt_grouped_gemm_tail_workspace_bytes(int dtype, int op, int32_t E, int64_t A, int64_t K,
                                             int64_t N);
@@ -418,8 +422,11 @@ int nt_grouped_gemm_dw(int dtype, const void* X, const int32_t* offsets, const v
  * When the dW has too few 256x256 tiles to fill the device and there are at
  * most 16 experts, one kernel launch runs both side by side (the dW on
  * 256x256 tiles, one per workgroup, the dX on the remaining CUs and then on
- * the dW's as they finish); otherwise they run one after the other. Outputs are bit-identical to the two separate calls. ws: the dW
- * workspace (nt_grouped_gemm_workspace_bytes). Replaces the pair of calls in
+ * the dW's as they finish); otherwise they run one after the other. ws: the dW
+ * workspace (nt_grouped_gemm_workspace_bytes), and where the dX is to be cut
+ * its own behind that (nt_grouped_gemm_tail_workspace_bytes). Outputs are
+ * bit-identical to the two separate calls: with the dW workspace alone to a dX
+ * without one, with both to a dX with its own. Replaces the pair of calls in
  * GroupedGEMM_FN.backward (reference
  * src/model/moe_ops.py:117-125; csrc/kernels/bwd_grouped_gemm_dW.cu:43-86,
  * bwd_grouped_gemm_dX.cu:46-96). */

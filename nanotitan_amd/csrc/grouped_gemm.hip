@@ -2097,10 +2097,14 @@ int pair_dw_dx(int dtype, const void* X, const int32_t* offsets, const void* dOu
   if (!pair) {
     const int st = dw_impl(dtype, X, offsets, dOut, E, A, K, N, dW, ws, ws_bytes, stream);
     if (st != NT_OK) return st;
-    // the dW and its reduce are done with the workspace (stream order)
-    const int tst = attach_tail(gx, EPIX == kEpiDualK ? NT_GEMM_DX2 : NT_GEMM_DX, dtype, ws,
-                                ws_bytes, stream);
-    if (tst != NT_OK) return tst;
+    // The dX is cut only with its own workspace behind the dW's: not in spare
+    // bytes of a dW workspace, whose caller's separate dX has none.
+    const size_t dw_bytes = round_up(nt_grouped_gemm_workspace_bytes(dtype, E, A, K, N), 256);
+    if (ws != nullptr && ws_bytes > dw_bytes) {
+      const int tst = attach_tail(gx, EPIX == kEpiDualK ? NT_GEMM_DX2 : NT_GEMM_DX, dtype,
+                                  static_cast<char*>(ws) + dw_bytes, ws_bytes - dw_bytes, stream);
+      if (tst != NT_OK) return tst;
+    }
     return launch_mode<kDx, EPIX>(dtype, gx, K, dx_mfma, stream);
   }
   GemmArgs gw{X, dOut, offsets, E, A, K, N, dW, 0, 0, 0, nullptr, nullptr, 0, nullptr};

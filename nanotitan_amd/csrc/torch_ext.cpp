@@ -86,11 +86,12 @@ size_t tail_workspace(const Tensor& like, int op, int32_t E, int64_t A, int64_t 
   return bytes;
 }
 
-// Of a dW + dX call: the larger of the dW's and its dX's.
+// Of a dW + dX call: the dW's, and behind it the dX's.
 Tensor pair_workspace(const Tensor& like, int op, int32_t E, int64_t A, int64_t K, int64_t N) {
   const int dt = dtype_code(like);
-  return workspace(like, std::max(nt_grouped_gemm_workspace_bytes(dt, E, A, K, N),
-                                  nt_grouped_gemm_tail_workspace_bytes(dt, op, E, A, K, N)));
+  const size_t dw = nt_grouped_gemm_workspace_bytes(dt, E, A, K, N);
+  const size_t tail = nt_grouped_gemm_tail_workspace_bytes(dt, op, E, A, K, N);
+  return workspace(like, tail > 0 ? (dw + 255) / 256 * 256 + tail : dw);
 }
 
 // ------------------------------------------------------ reference surface

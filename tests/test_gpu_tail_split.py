@@ -144,3 +144,43 @@ def test_fused_dx_equals_dx_where_dx_is_not_cut(ext, E, rows, K, N):
     assert torch.equal(dH, (dX.float() * H.float()).to(W.dtype))
     assert torch.equal(ext.bwd_grouped_gemm_dX_swiglu(W, offs, D, G, V)[1], 64 * dX)
     assert torch.equal(ext.bwd_grouped_gemm_dW_dX_gelu(H, W, offs, D, H)[1], dH)
+
+
+@pytest.mark.parametrize("dtype,K,N", [(torch.bfloat16, 512, 4096), (torch.float32, 300, 1001)])
+def test_dw_dx_follows_the_workspace_it_is_given(ext, dtype, K, N):
+    """The C ABI's dW + dX call equals a dX without a workspace when it has the
+    dW's alone (however large that is), and a dX with its own when it has both."""
+    code, lib, s = capi.dtype_code(dtype), capi.load(), capi.current_stream()
+    counts = [3900] + [350 + 11 * e for e in range(31)]  # more than 16: not paired
+    E, A = len(counts), sum(counts)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    offs = torch.tensor([0, *torch.tensor(counts).cumsum(0).tolist()], dtype=torch.int32,
+                        device="cuda")
+
+    def randn(*shape):
+        return torch.randn(shape, generator=g, device="cuda").to(dtype)
+
+    X, W, D = randn(A, K), randn(E, K, N), randn(A, N)
+    dw = lib.nt_grouped_gemm_workspace_bytes(code, E, A, K, N)
+    tail = lib.nt_grouped_gemm_tail_workspace_bytes(code, 1, E, A, K, N)
+    assert tail > 0 and (dw > tail or dtype == torch.float32)
+    ws = torch.empty(dw + 255 + tail, dtype=torch.uint8, device="cuda")
+
+    def dx(size):
+        out = torch.full_like(X, 7)
+        capi.call("nt_grouped_gemm_dx", code, capi.ptr(W), capi.ptr(offs), capi.ptr(D), E, A, K,
+                  N, capi.ptr(out), capi.ptr(ws) if size else None, size, s)
+        return out
+
+    def dw_dx(size):
+        out, dW = torch.full_like(X, 7), torch.empty_like(W)
+        capi.call("nt_grouped_gemm_dw_dx", code, capi.ptr(X), capi.ptr(W), capi.ptr(offs),
+                  capi.ptr(D), E, A, K, N, capi.ptr(dW), capi.ptr(out), capi.ptr(ws), size, s)
+        return out
+
+    whole, cut = dx(0), dx(tail)
+    assert not torch.equal(whole, cut)  # the sizes are cut
+    assert torch.equal(dw_dx(dw), whole)
+    assert torch.equal(dw_dx((dw + 255) // 256 * 256 + tail), cut)
+    assert torch.equal(ext.bwd_grouped_gemm_dX_kernel(W, offs, D), cut)
+    assert torch.equal(ext.bwd_grouped_gemm_dW_dX(X, W, offs, D)[1], cut)
