@@ -99,9 +99,6 @@ def family(name: str) -> str:
     m = re.search(r"gg_pair_kernel<[^,]+, (\d+)", name)
     if m:
         return "gemm_pair_dw_dx_gelu" if m.group(1) == "2" else "gemm_pair_dw_dx"
-    m = re.search(r"gg_f32_mfma_kernel<(\d+), (\d+)>", name)
-    if m:
-        return {"0": "gemm_fwd", "1": "gemm_dx", "2": "gemm_dw"}[m.group(1)]
     m = re.search(r"gg_staged_kernel<[^,]+, (\d+), (\d+)>", name)
     if m:
         return {"00": "gemm_fwd", "01": "gemm_fwd_gelu", "03": "gemm_fwd", "10": "gemm_dx",

@@ -192,3 +192,54 @@ def test_router_linear_backward_from_float32(ext, dtype, T, E, d, shift):
     assert bool(((got[1].cpu().double() - dld.t() @ xd).abs() <= bound).all())
     with pytest.raises(RuntimeError):  # only float32 tokens may differ from their gradient
         ext.router_linear_backward(x.cuda(), W, dl, None, True, True, torch.float32)
+
+
+class _Doubled(torch.nn.Linear):
+    def forward(self, x):
+        return 2 * super().forward(x)
+
+
+@pytest.mark.parametrize("change", ["none", "bias", "subclass", "bf16", "pre_hook", "backward_hook",
+                                    "backward_pre_hook", "global_hook", "instance_forward",
+                                    "autocast", "tensor_weight"])
+def test_only_a_plain_router_runs_once(ext, change):
+    """Any other router is called, twice, and its statistics are torch's."""
+    from nanotitan_amd.layer import _plain_router
+
+    moe, x = _moe(8)
+    r, handle, context = moe.router, None, torch.no_grad()
+    if change == "bias":
+        r.bias = torch.nn.Parameter(torch.randn(8, device="cuda"))
+    elif change == "subclass":
+        r.__class__ = _Doubled
+    elif change == "bf16":
+        r.to(torch.bfloat16)
+    elif change == "pre_hook":
+        handle = r.register_forward_pre_hook(lambda m, a: (a[0] * 3,))
+    elif change == "backward_hook":
+        handle = r.register_full_backward_hook(lambda *a: None)
+    elif change == "backward_pre_hook":
+        handle = r.register_full_backward_pre_hook(lambda *a: None)
+    elif change == "global_hook":
+        handle = torch.nn.modules.module.register_module_forward_hook(lambda *a: None)
+    elif change == "instance_forward":
+        r.forward = lambda t: torch.nn.functional.linear(t, r.weight) * 2
+    elif change == "autocast":
+        context = torch.autocast("cuda", dtype=torch.bfloat16)
+    elif change == "tensor_weight":
+        del r._parameters["weight"]
+        r.weight = torch.randn(8, 48, device="cuda")
+    try:
+        flat = x.reshape(-1, 48)
+        with context:
+            assert _plain_router(r, flat) == (change == "none")
+            _, st = moe(x)
+            probs = r(flat.to(r.weight.dtype)).softmax(dim=-1).float().mean(dim=0)
+        # the router's own logits: bf16 ones (and their mean) round to 8 bits
+        low = change in ("bf16", "autocast")
+        torch.testing.assert_close(st.probs_per_expert.float(), probs,
+                                   rtol=2.0**-7 if low else 2e-5, atol=2.0**-9 if low else 1e-6)
+        assert int(st.total_assignments) == 2 * flat.shape[0]
+    finally:
+        if handle is not None:
+            handle.remove()

@@ -184,3 +184,66 @@ def test_dw_dx_follows_the_workspace_it_is_given(ext, dtype, K, N):
     assert torch.equal(dw_dx((dw + 255) // 256 * 256 + tail), cut)
     assert torch.equal(ext.bwd_grouped_gemm_dX_kernel(W, offs, D), cut)
     assert torch.equal(ext.bwd_grouped_gemm_dW_dX(X, W, offs, D)[1], cut)
+
+
+UNEVEN = [1371, 0, 1203, 1280, 1, 2049, 1999, 1408, 900, 1155, 1666, 1537, 1024, 1290, 1811, 1300]
+
+
+@pytest.mark.parametrize("dtype,op,K,N,scale", [
+    (torch.bfloat16, "fwd", 4096, 512, 1), (torch.float16, "dx2", 512, 2048, 1.6),
+    (torch.bfloat16, "dx2", 512, 2112, 1)])
+def test_whole_tiles_then_pieces(ext, dtype, op, K, N, scale):
+    """More tiles than workgroups: a workgroup multiplies whole tiles first and
+    loads its piece of the last round behind their stores. The same bounds; the
+    uncut tiles' bits; run to run; and under graph replay."""
+    counts = [int(c * scale) for c in UNEVEN]
+    E, A = len(counts), sum(counts)
+    assert sum(-(-c // 128) for c in counts) * 4 > 512  # 512 columns; two workgroups per CU
+    g = torch.Generator(device="cuda").manual_seed(N)
+    offs = torch.tensor([0, *torch.tensor(counts).cumsum(0).tolist()], dtype=torch.int32,
+                        device="cuda")
+    seg = [(e, slice(int(offs[e]), int(offs[e + 1]))) for e in range(E)]
+    R = K if op == "fwd" else N  # reduction of one part
+
+    def randn(*shape):
+        return torch.randn(shape, generator=g, device="cuda").to(dtype)
+
+    a = [randn(A, R) for _ in range(1 if op == "fwd" else 2)]
+    W = [randn(E, K, N) for _ in a]
+
+    def call():
+        if op == "fwd":
+            return ext.grouped_gemm_kernel(a[0], offs, W[0])
+        return ext.bwd_grouped_gemm_dX2(*W, offs, *a)
+
+    whole = call()
+    args = [capi.dtype_code(dtype)]
+    if op == "fwd":
+        args += [capi.ptr(a[0]), capi.ptr(offs), capi.ptr(W[0])]
+    else:
+        args += [capi.ptr(W[0]), capi.ptr(W[1]), capi.ptr(offs), capi.ptr(a[0]), capi.ptr(a[1])]
+    capi.call("nt_grouped_gemm" if op == "fwd" else "nt_grouped_gemm_dx2", *args, E, A, K, N,
+              capi.ptr(whole), None, 0, capi.current_stream())
+
+    out = call()
+    assert not torch.equal(out, whole)  # some tiles are cut
+    assert float((out == whole).float().mean()) > 0.9  # single roundings differ
+
+    def rows(f):
+        return torch.cat([sum(f(x[s].double()) @ f(w[e].double() if op == "fwd" else
+                                                  w[e].double().t().contiguous())
+                              for x, w in zip(a, W)) for e, s in seg]).cpu()
+
+    ref, mag = rows(lambda t: t), rows(torch.abs)
+    _check(out, ref, mag, R * len(a), dtype)
+    _check(whole, ref, mag, R * len(a), dtype)
+    assert torch.equal(call(), out)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        again = call()
+    for _ in range(3):
+        a[0].copy_(randn(A, R))
+        graph.replay()
+        eager = call()
+        torch.cuda.synchronize()
+        assert torch.equal(again, eager)

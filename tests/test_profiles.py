@@ -76,8 +76,10 @@ def test_kernel_families():
                   "(nt::GemmArgs)") == "gemm_dx_gelu"
     assert family("void nt::gg_pair_kernel<nt::bf16, 2, false>(nt::GemmArgs, nt::GemmArgs, int, "
                   "int*)") == "gemm_pair_dw_dx_gelu"
-    assert family("void nt::(anonymous namespace)::gg_f32_mfma_kernel<2, 0>(nt::GemmArgs)") \
+    assert family("void nt::(anonymous namespace)::gg_staged_kernel<float, 2, 0>(nt::GemmArgs)") \
         == "gemm_dw"
+    assert family("void nt::(anonymous namespace)::gg_mfma_tail_kernel<nt::bf16, 1, 5>"
+                  "(nt::GemmArgs)") == "gemm_dx"
     assert family("void nt::pack_rows_kernel<HIP_vector_type<unsigned int, 4u> >(...)") \
         == "dispatch_pack"
     assert family("void nt::combine_bwd_inv_kernel<nt::bf16, nt::bf16, 8, 2>(...)") == "combine_bwd"
