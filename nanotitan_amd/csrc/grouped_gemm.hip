@@ -895,8 +895,8 @@ __device__ __forceinline__ void gemm_tiles(const GemmArgs& g, int64_t wg, int64_
   const int64_t t_beg = MODE == kDw ? total * before / G
                                     : xcd_range_start(total, before, G, s_pref, g.E, g.ntn);
   int64_t logical = t_beg + wg / kXcd;
-  // Tail split: tiles from t_full on are np workgroups each; tile_range gives
-  // this workgroup's k-steps of the tile it takes at `t`, and the tile.
+  // Tail split: tiles from t_full on are np workgroups each; tail_item gives
+  // the tile of the item at `t` and this workgroup's piece of it.
   int64_t t_full = t_end;
   int np = 1, piece = 0;
   if constexpr (TAIL) {
@@ -1527,7 +1527,25 @@ constexpr int64_t kFewRows = 32, kFewRowsSwiGLU = 48;
 //                      SwiGLU    460 -> 390  467 -> 400  474 -> 409  487 -> 527
 //    16,  512 -> 2048  up         12 ->  14   12 ->  14   12 ->  15
 //                      SwiGLU     27 ->  20   27 ->  20   27 ->  20   27 ->  32
-// (the last layer's weights stay in the cache: only its SwiGLU gains).
+// (the last layer's weights stay in the cache: only its SwiGLU gains). With
+// routed counts (uniform routing, top-8 of 128, top-2 of the others) a few
+// experts pass 128 rows from a mean of about 105 on:
+//                        mean rows   64          96          112
+//   128, 2048 ->  768  up         90 ->  89   93 ->  93  100 ->  93
+//                      down       88 ->  87  104 ->  91  107 -> 102
+//                      SwiGLU    192 -> 162  197 -> 167  202 -> 198
+//     8, 4096 -> 14336 up        188 -> 174  196 -> 177  197 -> 176
+//                      down      236 -> 227  256 -> 231  259 -> 238
+//                      SwiGLU    460 -> 393  465 -> 406  471 -> 407
+//    16,  512 -> 2048  SwiGLU     27 ->  20   27 ->  20   26 ->  20 or 31
+// (the last: 16 experts x 16 column tiles are one round of the CUs, and one
+// expert past 128 rows makes it two). The rules know only the mean: where most
+// experts are empty the rest have many row tiles, for which the taller tiles
+// before can be the better ones (all rows of a mean of 32 in 4 of 128 experts:
+// up 768 -> 2048 19 -> 28, its SwiGLU 35 -> 57, 2048 -> 768 29 -> 28 and
+// 59 -> 58; in 4 of 8 experts 4096 -> 14336 92 -> 82 and 234 -> 187); under
+// Zipf-skewed counts (exponent 1.2) the two larger layers take 0.6 to 1.33 of
+// the time before, most of them less than it.
 constexpr int64_t kMidRows = 112;
 constexpr int64_t kStreamedBytes = int64_t(256) << 20;
 // The tile rules of forward and dX launches, shared with the tail split's

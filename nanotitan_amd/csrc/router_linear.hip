@@ -5,11 +5,12 @@
 //
 // All of it is small next to the experts, so launches and passes over the
 // tokens are what it costs: on MI355X, 16,384 tokens x 512, 16 experts, the
-// library's two fp32 dW products alone took 150 us (its tiles hold 16 of
+// library's two fp32 dW products alone took 149 us (its tiles hold 16 of
 // their output columns) and dx, casts, sums and the second linear pass
-// another 80; the linear backward here takes 35 us and its reduce 5. The
+// another 80; the linear backward here takes 35 us for the gate path (dx and
+// dW) and 20 for the statistics path (dW), and each one's reduce 5. The
 // statistics were ten short launches (softmax, mean, sum, divide, ...): a
-// four-token forward, bound by the host, went from 188 to 118 us.
+// four-token forward, bound by the host, went from 194 to 118 us.
 #include <algorithm>
 
 #include "common.hpp"
@@ -314,8 +315,12 @@ struct LinearPlan {
   int vec, cg, nsub, groups;
   int64_t blocks, cols;
 };
-// Up to 512 workgroups along the tokens: enough to fill the chip, few
-// enough that their partial sums stay a small part of x's bytes.
+// Up to 512 workgroups along the tokens: enough to fill the chip, and a bound
+// on their partial sums. A workgroup of 64 tokens writes nsub E d floats, so
+// up to 32,768 tokens the partials are nsub E / 64 of float32 x's bytes (a
+// quarter at 16,384 x 512 and 16 experts, all of them at 128 columns, where
+// nsub is 4), less above. They are written and read once more; at 32,768 x
+// 8,192 and 32 experts they take 512 MiB of workspace.
 LinearPlan linear_plan(int64_t T, int64_t d, int vec) {
   LinearPlan p;
   p.vec = vec;
