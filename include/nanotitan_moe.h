@@ -344,7 +344,8 @@ int nt_grouped_gemm_dx(int dtype, const void* W, const int32_t* offsets, const v
                        size_t ws_bytes, hipStream_t stream);
 
 /* Up-projection with the GELU (erf form) fused into the epilogue. With
- * h = X_e @ W[e] rounded to dtype (as nt_grouped_gemm writes it), stores
+ * h = X_e @ W[e] rounded to dtype (the bits of nt_grouped_gemm without a
+ * workspace: a forward with a fused activation is never cut), stores
  * act = gelu(h) and act_grad = gelu'(h), both [A,N] and rounded once; h
  * itself is not stored (the backward needs only act_grad). The reference
  * runs grouped_gemm_kernel and then the activation
@@ -355,8 +356,9 @@ int nt_grouped_gemm_gelu(int dtype, const void* X, const int32_t* offsets, const
                          void* ws, size_t ws_bytes, hipStream_t stream);
 
 /* dX GEMM with the GELU backward fused into the epilogue:
- * dH = (dOut @ W[e]^T, rounded) * act_grad, rounded once, with act_grad the
- * gelu'(h) nt_grouped_gemm_gelu stored. W [E,K,N], dOut [A,N], act_grad and
+ * dH = (dOut @ W[e]^T, rounded: the bits of nt_grouped_gemm_dx with the same
+ * workspace) * act_grad, rounded once, with act_grad the gelu'(h)
+ * nt_grouped_gemm_gelu stored. W [E,K,N], dOut [A,N], act_grad and
  * dH [A,K]. Replaces bwd_grouped_gemm_dX_kernel followed by the
  * activation's backward (reference csrc/kernels/bwd_grouped_gemm_dX.cu:46-96,
  * then autograd). */
@@ -367,8 +369,9 @@ int nt_grouped_gemm_dx_gelu(int dtype, const void* W, const int32_t* offsets, co
 /* SwiGLU up-projection: the gate and value GEMMs of each output tile run
  * in one kernel (the B tiles of W_gate and W_val side by side) and the
  * epilogue writes gate = X_e @ W_gate[e], value = X_e @ W_val[e] (each
- * rounded to dtype) and hidden = silu(gate) * value (silu rounded, then the
- * product rounded), all [A,N]; gate and value are what the backward needs.
+ * rounded to dtype, the bits of nt_grouped_gemm without a workspace) and
+ * hidden = silu(gate) * value (silu rounded, then the product rounded), all
+ * [A,N]; gate and value are what the backward needs.
  * W_gate, W_val [E,K,N]. Replaces the two grouped_gemm_kernel calls and the
  * activation of the reference's SwiGLU ExpertFFN
  * (src/model/feed_fwd.py:107-110). */

@@ -2035,8 +2035,10 @@ bool pair_shape(int32_t E, int64_t K, int64_t N, int64_t cus) {
 // stay those of the activation applied to the separate dX: the rule is that
 // of the plain dX, also at few rows per expert, where a fused one runs on
 // 128x128 tiles like these but the plain one on 64-row tiles, never cut.
-// The GEMMs of wide outputs stay whole, so the SwiGLU forward's gate and
-// value are the separate GEMMs' bits there. Measured on MI355X, whole tiles
+// Forwards with a fused activation stay whole: the SwiGLU forward's gate and
+// value are the separate GEMMs' bits where those are not cut, which GEMMs of
+// outputs as wide as their reduction (the usual up projections) never are.
+// Measured on MI355X, whole tiles
 // to cut: bf16, two-part dX over 2 x 2048 to 512 for 16 experts: 4,096 rows
 // 49 to 40 us, 32,768 rows 157 to 144; down 14336 -> 4096 for 8 experts,
 // 4,096 rows 727 to 593. fp32, down 2048 -> 512 for 8 experts: 1,040 rows 117

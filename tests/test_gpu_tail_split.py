@@ -247,3 +247,24 @@ def test_whole_tiles_then_pieces(ext, dtype, op, K, N, scale):
         eager = call()
         torch.cuda.synchronize()
         assert torch.equal(again, eager)
+
+
+@pytest.mark.parametrize("dtype,K,N", [(torch.bfloat16, 4096, 136), (torch.float32, 512, 130),
+                                       (torch.bfloat16, 1365, 300)])
+def test_fused_forward_holds_the_bits_of_whole_tiles(ext, dtype, K, N):
+    """An up projection narrower than its input: the plain forward is cut with a
+    workspace, the fused ones never are."""
+    offs, X, W, _ = _case(dtype, K, N)
+    A, E = X.shape[0], W.shape[0]
+    og, Xg, Wg = offs.cuda(), X.cuda(), W.cuda()
+    Vg = Wg.flip(2).contiguous()
+
+    def whole(w):
+        out = torch.empty(A, N, dtype=dtype, device="cuda")
+        capi.call("nt_grouped_gemm", capi.dtype_code(dtype), capi.ptr(Xg), capi.ptr(og),
+                  capi.ptr(w), E, A, K, N, capi.ptr(out), None, 0, capi.current_stream())
+        return out
+
+    assert not torch.equal(ext.grouped_gemm_kernel(Xg, og, Wg), whole(Wg))  # cut
+    _, gate, value = ext.grouped_gemm_swiglu(Xg, og, Wg, Vg)
+    assert torch.equal(gate, whole(Wg)) and torch.equal(value, whole(Vg))
